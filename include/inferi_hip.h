@@ -102,15 +102,15 @@ IFR_API ifr_status ifr_device_info(ifr_ctx *ctx, char *name, size_t name_len, in
  * "pf_chunk"
  * sets the prompt tokens per ifr_llama2_prefill pass (a multiple of 64, at
  * most 16384; 0 = 4096), read at a state's first prefill.  "pf_tile"
- * selects the prefill GEMM's tiles: 0 (the default) 256 x 256 tiles where a
- * product has at least 128 of them, else 128 x 128 tiles; 128 or 256 forces
- * one form.  "pf_ws" = 1 (the default) runs the Q4_K products on 256 x 256
- * tiles in the warp-specialized form (eight MFMA waves and four waves that
- * load and dequantize the tiles), 0 in the eight-wave form where every wave
- * does both.  Every form sums each output element's products in the same
+ * selects the prefill GEMM's tiles: 0 (the default) the smallest of 32 x 32,
+ * 64 x 64, 128 x 128 and 256 x 256 whose tiles the chip runs at once; 128 or
+ * 256 forces that one.  "pf_ws" = 1 (the default) runs the Q4_K products on
+ * 256 x 256 tiles in the warp-specialized form (eight MFMA waves and four
+ * waves that load and dequantize the tiles; other types always do), 0 in the
+ * eight-wave form where every wave does both.  Every form sums each output element's products in the same
  * order, so the results do not depend on the form or the pass length.
- * "pf_rope_fuse" = 1 (the default) lets the warp-specialized Q/K/V product
- * add the biases, apply RoPE and store k and v to the cache in its epilogue
+ * "pf_rope_fuse" = 1 (the default) lets the Q/K/V product (three matrices of
+ * one type; not in the eight-wave form) add the biases, apply RoPE and store k and v to the cache in its epilogue
  * (pairs (2i, 2i + 1) only), 0 leaves that to a kernel of its own; both
  * give the same results bit for bit.
  * A captured decode step is captured again after any option change. */

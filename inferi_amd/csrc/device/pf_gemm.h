@@ -19,9 +19,11 @@
 // loads, issued a step ahead; W's GGUF bytes arrive in registers two steps
 // ahead and are dequantized into the other buffer while the matrix cores
 // work on the current one, so one barrier per step suffices.  (Four waves
-// of 128 x 128, one per SIMD, measured 10-20% slower.)  Q4_K products take
-// a warp-specialized form of the same tile (pf_gemm_ws_body, below), where
-// four more waves do all the loading and dequantizing.
+// of 128 x 128, one per SIMD, measured 10-20% slower.)  That is the eight-wave
+// form, Q4_K's with option pf_ws = 0.  By default the products take a
+// warp-specialized form of the same tile, where four more waves do all the
+// loading and dequantizing: pf_gemm_ws_body (Q4_K) and pf_gemm_wr_body (the
+// other types); device/pf_small.h has the smaller tiles.
 //
 // Rows of the virtual n range come from up to three matrices of one GGUF
 // type stacked one after another (n < n1: w0, n < n2: w1, else w2), so Q, K
@@ -35,7 +37,7 @@
 // rounded division took about 25 VALU instructions per value, 64 values per
 // lane at the end of every tile while the matrix cores idle).
 #pragma once
-#include "pf_tiles.h"
+#include "pf_runs.h"
 
 namespace ifr {
 
@@ -46,17 +48,6 @@ constexpr int PG_THREADS = 512;
 constexpr int PG_STORE = 0;  // Y = X W^T
 constexpr int PG_ADD = 1;    // Y += X W^T (the residual stream)
 constexpr int PG_SWIGLU = 2; // h = f16(up * silu(gate)), gate/up interleaved by 32 rows
-
-// LDS tiles: 256 rows of 64 halves (128 B) without padding; the 16-byte
-// chunk c of row r sits at chunk c ^ s(r), s(r) = ((r / 2) ^ 4 (r % 2)) % 8.
-// The sixteen consecutive rows whose 16-byte chunks one read pass serves (64
-// banks of 4 bytes, two rows per bank line) fall on distinct banks; the
-// dequantized row stores, two threads per row, meet fewer conflicts than
-// with s(r) = (r / 2) % 8 (a microbenchmark of the two access patterns:
-// reads 5.1 -> 4.7, stores 16.0 -> 14.1 cycles per wave instruction and CU;
-// the 4095-token 8B prefill 69.4 -> 69.1 ms, alternated three times).
-IFR_DEV uint32_t pg_swz_of(uint32_t r) { return ((r >> 1) ^ ((r & 1u) << 2)) & 7u; }
-IFR_DEV uint32_t pg_swz(uint32_t r, uint32_t c) { return r * PG_BK + 8 * (c ^ pg_swz_of(r)); }
 
 typedef __attribute__((address_space(3))) char lds_char_t;
 
@@ -80,40 +71,6 @@ IFR_DEV void lds_dma16(const void *base, uint32_t off, uint32_t lds) {
 // wait tracking): the caller waits with s_waitcnt before reading r.
 IFR_DEV void ld16_asm(u32x4_a16 &r, const uint8_t *p) { asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(r) : "v"(p)); }
 
-// Weight staging of one thread: half (part p) of one tile row's 64 elements
-// in a K step, stored as four swizzled 16-byte chunks.  Generic: the PfTile
-// loader's elements [32 p, +32) (chunks 4p .. 4p + 3), with compiler-tracked
-// loads.
-template <int FMT>
-struct PgHalf {
-    static constexpr bool MANUAL = false;
-    PfTile<FMT> t;
-    IFR_DEV void load(const uint8_t *wrow, uint32_t k0, uint32_t p) { t.load(wrow, k0, p); }
-    template <int N>
-    IFR_DEV void wait() {}
-    IFR_DEV void store(uint32_t k0, uint32_t p, _Float16 *tile, uint32_t r) const {
-        _Float16 h[32];
-        t.deq(k0, p, h);
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            uint4 u;
-            __builtin_memcpy(&u, &h[8 * c], 16);
-            *(uint4 *)(tile + pg_swz(r, 4 * p + (uint32_t)c)) = u;
-        }
-    }
-};
-// The block affine map of the step's two sub-blocks 2g, 2g + 1 (g = (k0 %
-// 256) / 64): y = d1 q + n1 (low nibbles), d2 q + n2 (high nibbles).
-struct Q4kAffine {
-    float d1, n1, d2, n2;
-};
-IFR_DEV Q4kAffine q4k_affine(const u32x4_a16 &hv, uint32_t k0) {
-#pragma clang fp contract(off)
-    uint32_t sc0, m0s, sc1, m1s;
-    scale_min_pair((k0 % 256) / 64, hv.y, hv.z, hv.w, sc0, m0s, sc1, m1s);
-    const float d = f16_to_f32(hv.x & 0xFFFFu), dm = f16_to_f32(hv.x >> 16);
-    return Q4kAffine{d * (float)sc0, -(dm * (float)m0s), d * (float)sc1, -(dm * (float)m1s)};
-}
 // The 16 qs bytes of part p (bytes [32 g + 16 p, +16) of the block's qs):
 // low nibbles -> chunks 2p, 2p + 1, high nibbles -> chunks 4 + 2p, 5 + 2p of
 // tile row r.
@@ -149,9 +106,9 @@ IFR_DEV void q4k_store_part(const u32x4_a16 &qv, const Q4kAffine &f, uint32_t p,
 // rounding, with the code's conversion folded into the mixed-precision FMA
 // (v_fma_mix_f32 reads the half in place).  Masks take two codes per
 // instruction, one in each half; f16 subnormal inputs are kept (the default
-// f16 denormal mode).
-typedef _Float16 f16x2v __attribute__((ext_vector_type(2)));
-IFR_DEV void q4k_store_part_mix(const u32x4_a16 &qv, const Q4kAffine &f, uint32_t p, _Float16 *tile, uint32_t r) {
+// f16 denormal mode).  x exchanges chunks (device/pf_small.h).
+IFR_DEV void q4k_store_part_mix(const u32x4_a16 &qv, const Q4kAffine &f, uint32_t p, _Float16 *tile, uint32_t r,
+                                uint32_t x = 0) {
     const float dl = f.d1 * 0x1p24f, dh = f.d2 * 0x1p20f; // exact: powers of two
     const uint32_t q[4] = {qv.x, qv.y, qv.z, qv.w};
     uint32_t lo[8], hi[8];
@@ -168,13 +125,11 @@ IFR_DEV void q4k_store_part_mix(const u32x4_a16 &qv, const Q4kAffine &f, uint32_
     }
 #pragma unroll
     for (int c = 0; c < 2; c++) {
-        *(uint4 *)(tile + pg_swz(r, 2 * p + (uint32_t)c)) = make_uint4(lo[4 * c], lo[4 * c + 1], lo[4 * c + 2], lo[4 * c + 3]);
-        *(uint4 *)(tile + pg_swz(r, 4 + 2 * p + (uint32_t)c)) = make_uint4(hi[4 * c], hi[4 * c + 1], hi[4 * c + 2], hi[4 * c + 3]);
+        *(uint4 *)(tile + pg_swz(r, (2 * p + (uint32_t)c) ^ x)) = make_uint4(lo[4 * c], lo[4 * c + 1], lo[4 * c + 2], lo[4 * c + 3]);
+        *(uint4 *)(tile + pg_swz(r, (4 + 2 * p + (uint32_t)c) ^ x)) = make_uint4(hi[4 * c], hi[4 * c + 1], hi[4 * c + 2], hi[4 * c + 3]);
     }
 }
-template <>
-struct PgHalf<Q4_K> {
-    static constexpr bool MANUAL = true;
+struct PgHalfQ4K {
     u32x4_a16 hv, qv;
     IFR_DEV void load(const uint8_t *wrow, uint32_t k0, uint32_t p) {
         const uint8_t *b = wrow + (size_t)(k0 / 256) * 144;
@@ -212,14 +167,13 @@ struct PgRowQ4K {
 };
 
 // One workgroup's state over the K loop.
-template <int FMT>
 struct PgCtx {
     _Float16 *xs[2], *ws[2];
     const _Float16 *x;
     uint32_t xoff[4];            // this lane's X rows of its four direct loads
     const uint8_t *wrow;
     uint32_t r, p, nk, lane, wave, wm, wn;
-    PgHalf<FMT> st0, st1;
+    PgHalfQ4K st0, st1;
     float16v acc[4][2];
 
     // X of step k into buffer B: four 1 KB direct loads per wave (lane l of
@@ -259,16 +213,13 @@ struct PgCtx {
     // 2 weight loads of this step.
     template <int B>
     IFR_DEV void step(uint32_t s) {
-        PgHalf<FMT> &ld = B ? st1 : st0, &dq = B ? st0 : st1;
+        PgHalfQ4K &ld = B ? st1 : st0, &dq = B ? st0 : st1;
         load_x<B ^ 1>(min(s + 1, nk - 1));
         ld.load(wrow, min(s + 2, nk - 1) * PG_BK, p);
-        dq.template wait<6>();
+        dq.wait<6>();
         dq.store(min(s + 1, nk - 1) * PG_BK, p, ws[B ^ 1], r);
         mfma_step<B>();
-        if constexpr (PgHalf<FMT>::MANUAL)
-            asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        else
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
 };
 
@@ -300,14 +251,15 @@ IFR_DEV const uint8_t *pg_wrow(const PfGemmArgs &a, uint32_t n0, uint32_t r) {
     }
 }
 
-// One wave's (32 MI) x 64 share of the tile out of its accumulators.
+// One wave's (32 MI) x (32 NJ) share of the tile out of its accumulators.
 // D[row][col] of block (i, j): col = lane % 32 (n), row = 8 (e / 4) + 4 (lane
 // / 32) + e % 4 (m).
-template <int EPI, int MI = 4>
-IFR_DEV void pg_epilogue(const PfGemmArgs &a, const float16v (&acc)[MI][2], uint32_t lane, uint32_t wm, uint32_t wn,
+template <int EPI, int MI = 4, int NJ = 2>
+IFR_DEV void pg_epilogue(const PfGemmArgs &a, const float16v (&acc)[MI][NJ], uint32_t lane, uint32_t wm, uint32_t wn,
                          uint32_t m0, uint32_t n0) {
     const uint32_t li = lane & 31u;
     if constexpr (EPI == PG_SWIGLU) {
+        static_assert(NJ == 2, "gate and up of an output in one lane");
         const uint32_t jn = n0 / 2 + wn / 2 + li;
         if (jn >= a.n1) return;
 #pragma unroll
@@ -327,7 +279,7 @@ IFR_DEV void pg_epilogue(const PfGemmArgs &a, const float16v (&acc)[MI][2], uint
         // element behind each element's bounds branch (the O and down
         // products' epilogue, 67 MB read and written at the 8B shape).
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
+        for (int j = 0; j < NJ; j++) {
             const uint32_t n = n0 + wn + 32 * j + li;
             if (n >= a.N) continue;
 #pragma unroll
@@ -356,13 +308,13 @@ IFR_DEV void pg_epilogue(const PfGemmArgs &a, const float16v (&acc)[MI][2], uint
     }
 }
 
-template <int FMT, int EPI>
+template <int EPI>
 __device__ __attribute__((always_inline)) void pf_gemm_body(const PfGemmArgs &a) {
     // four LDS objects, so the compiler sees that the direct loads into one
     // buffer do not alias the operand reads of the other
     __shared__ __attribute__((aligned(1024))) _Float16 xs0[PG_BM * PG_BK], xs1[PG_BM * PG_BK];
     __shared__ __attribute__((aligned(1024))) _Float16 ws0[PG_BN * PG_BK], ws1[PG_BN * PG_BK];
-    PgCtx<FMT> g;
+    PgCtx g;
     const uint32_t tid = threadIdx.x;
     g.xs[0] = xs0;
     g.xs[1] = xs1;
@@ -400,25 +352,19 @@ __device__ __attribute__((always_inline)) void pf_gemm_body(const PfGemmArgs &a)
 
     // prologue: X and weights of step 0 into buffer 0, weights of step 1 in
     // flight
-    g.template load_x<0>(0);
+    g.load_x<0>(0);
     g.st0.load(g.wrow, 0, g.p);
     g.st1.load(g.wrow, min(1u, g.nk - 1) * PG_BK, g.p);
-    g.st0.template wait<2>();
+    g.st0.wait<2>();
     g.st0.store(0, g.p, ws0, r);
-    if constexpr (PgHalf<FMT>::MANUAL)
-        asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    else
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     for (uint32_t s = 0; s < g.nk; s += 2) {
-        g.template step<0>(s);
-        if (s + 1 < g.nk) g.template step<1>(s + 1);
+        g.step<0>(s);
+        if (s + 1 < g.nk) g.step<1>(s + 1);
     }
     // the clamped loads past the end: their destination registers stay
     // allocated until they have landed
-    if constexpr (PgHalf<FMT>::MANUAL)
-        asm volatile("s_waitcnt vmcnt(0)" : "+v"(g.st0.hv), "+v"(g.st0.qv), "+v"(g.st1.hv), "+v"(g.st1.qv)::"memory");
-    else
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(g.st0.hv), "+v"(g.st0.qv), "+v"(g.st1.hv), "+v"(g.st1.qv)::"memory");
     pg_epilogue<EPI>(a, g.acc, g.lane, g.wm, g.wn, m0, n0);
 }
 
@@ -432,19 +378,19 @@ __device__ __attribute__((always_inline)) void pf_gemm_body(const PfGemmArgs &a)
 // from the pass's table; q goes to Y, k and v to the cache rows of positions
 // p0 + m.  Eight rows at a time: their table loads go out together from
 // rows clamped below M.
-template <int MI>
-IFR_DEV void pg_epilogue_rope(const PfGemmArgs &a, const float16v (&acc)[MI][2], uint32_t lane, uint32_t wm,
+template <int MI, int NJ = 2>
+IFR_DEV void pg_epilogue_rope(const PfGemmArgs &a, const float16v (&acc)[MI][NJ], uint32_t lane, uint32_t wm,
                               uint32_t wn, uint32_t m0, uint32_t n0) {
     constexpr int RB = 4; // rows per batch
     const uint32_t li = lane & 31u, odd = lane & 1u, hh = a.head_size / 2, kd = a.n2 - a.n1;
     // per column block j: the column, its vector (0 q, 1 k, 2 v), element,
     // bias and table column
-    bool nok[2];
-    uint32_t n[2], seg[2], e[2], tj[2];
-    float bv[2];
-    bool hb[2];
+    bool nok[NJ];
+    uint32_t n[NJ], seg[NJ], e[NJ], tj[NJ];
+    float bv[NJ];
+    bool hb[NJ];
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
+    for (int j = 0; j < NJ; j++) {
         n[j] = n0 + wn + 32 * j + li;
         nok[j] = n[j] < a.N; // the same for both lanes of a pair
         const uint32_t nc = nok[j] ? n[j] : a.N - 1;
@@ -476,21 +422,21 @@ IFR_DEV void pg_epilogue_rope(const PfGemmArgs &a, const float16v (&acc)[MI][2],
 #pragma unroll
         for (int h = 0; h < 16; h += RB) {
             uint32_t m[RB];
-            float cs[2][RB], sn[2][RB];
+            float cs[NJ][RB], sn[NJ][RB];
 #pragma unroll
             for (int q = 0; q < RB; q++) {
                 const int ee = h + q;
                 m[q] = m0 + wm + 32 * i + 8 * (ee / 4) + 4 * (lane >> 5) + (ee % 4);
                 const uint32_t rowt = min(m[q], a.M - 1) * hh;
 #pragma unroll
-                for (int j = 0; j < 2; j++) {
+                for (int j = 0; j < NJ; j++) {
                     const float2 t = *(const float2 *)((const char *)a.rope_cs + 8u * (rowt + tj[j]));
                     cs[j][q] = t.x;
                     sn[j][q] = t.y;
                 }
             }
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+            for (int j = 0; j < NJ; j++)
 #pragma unroll
                 for (int q = 0; q < RB; q++) {
                     float v = acc[i][j][h + q];
@@ -618,8 +564,8 @@ __device__ __attribute__((always_inline)) void pf_gemm_ws_half(const PfGemmArgs 
         for (int j = 0; j < 8; j++) lds_dma16(x + k * PG_BK, xoff[j], __builtin_amdgcn_readfirstlane(dst + 1024 * j));
     };
     const uint8_t *wrow = pg_wrow<EPI>(a, n0, r);
-    PgHalf<Q4_K> st0, st1;
-    auto store = [&](const PgHalf<Q4_K> &st, uint32_t k0, _Float16 *tile) {
+    PgHalfQ4K st0, st1;
+    auto store = [&](const PgHalfQ4K &st, uint32_t k0, _Float16 *tile) {
         q4k_store_part_mix(st.qv, q4k_affine(st.hv, k0), p, tile, r);
     };
     // as the whole tile's staging with two weight loads per step: in
@@ -628,19 +574,19 @@ __device__ __attribute__((always_inline)) void pf_gemm_ws_half(const PfGemmArgs 
     load_x(xdst0, 0);
     st0.load(wrow, 0, p);
     st1.load(wrow, min(1u, nk - 1) * PG_BK, p);
-    st0.template wait<2>();
+    st0.wait<2>();
     store(st0, 0, ws0);
     asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     for (uint32_t s = 0; s < nk; s += 2) {
         load_x(xdst1, min(s + 1, nk - 1));
         st0.load(wrow, min(s + 2, nk - 1) * PG_BK, p);
-        st1.template wait<10>();
+        st1.wait<10>();
         store(st1, min(s + 1, nk - 1) * PG_BK, ws1);
         asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if (s + 1 < nk) {
             load_x(xdst0, min(s + 2, nk - 1));
             st1.load(wrow, min(s + 3, nk - 1) * PG_BK, p);
-            st0.template wait<10>();
+            st0.wait<10>();
             store(st0, min(s + 2, nk - 1) * PG_BK, ws0);
             asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         }
@@ -677,7 +623,7 @@ __device__ __attribute__((always_inline)) void pf_gemm_ws_body(const PfGemmArgs 
     if (wave < 8) {
         // MFMA waves
         const uint32_t wm = 128 * (wave & 1u), wn = 64 * (wave >> 1);
-        PgCtx<Q4_K> g;
+        PgCtx g;
         g.lane = lane;
         g.wm = wm;
         g.wn = wn;
@@ -693,10 +639,10 @@ __device__ __attribute__((always_inline)) void pf_gemm_ws_body(const PfGemmArgs 
                 for (int e = 0; e < 16; e++) g.acc[i][j][e] = 0.0f;
         asm volatile("s_barrier" ::: "memory");
         for (uint32_t s = 0; s < nk; s += 2) {
-            g.template mfma_step<0>();
+            g.mfma_step<0>();
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
             if (s + 1 < nk) {
-                g.template mfma_step<1>();
+                g.mfma_step<1>();
                 asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
             }
         }
@@ -730,7 +676,7 @@ __device__ __attribute__((always_inline)) void pf_gemm_ws_body(const PfGemmArgs 
     load_x(xdst0, 0);
     st0.load(wrow, 0);
     st1.load(wrow, min(1u, nk - 1) * PG_BK);
-    st0.template wait<3>();
+    st0.wait<3>();
     st0.store(0, ws0, t);
     asm volatile("s_waitcnt vmcnt(3) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     // step s: X of step s + 1 (8 loads) and the weights of step s + 2 (3)
@@ -742,13 +688,13 @@ __device__ __attribute__((always_inline)) void pf_gemm_ws_body(const PfGemmArgs 
     for (uint32_t s = 0; s < nk; s += 2) {
         load_x(xdst1, min(s + 1, nk - 1));
         st0.load(wrow, min(s + 2, nk - 1) * PG_BK);
-        st1.template wait<11>();
+        st1.wait<11>();
         st1.store(min(s + 1, nk - 1) * PG_BK, ws1, t);
         asm volatile("s_waitcnt vmcnt(3) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if (s + 1 < nk) {
             load_x(xdst0, min(s + 2, nk - 1));
             st1.load(wrow, min(s + 3, nk - 1) * PG_BK);
-            st0.template wait<11>();
+            st0.wait<11>();
             st0.store(min(s + 2, nk - 1) * PG_BK, ws0, t);
             asm volatile("s_waitcnt vmcnt(3) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         }
@@ -757,6 +703,133 @@ __device__ __attribute__((always_inline)) void pf_gemm_ws_body(const PfGemmArgs 
     // allocated until they have landed
     asm volatile("s_waitcnt vmcnt(0)" : "+v"(st0.hv), "+v"(st0.q0), "+v"(st0.q1), "+v"(st1.hv), "+v"(st1.q0),
                  "+v"(st1.q1)::"memory");
+}
+
+// The warp-specialized form for every type, on PgRun: as pf_gemm_ws_body, but
+// the MFMA waves request X themselves (four direct loads each, a step ahead),
+// so that the staging waves' queue holds only weight loads, which the
+// compiler tracks by itself.  A whole tile's staging thread owns a row's two
+// runs, a half tile's one of them.  On Q4_K it measured 1-3.5% slower than
+// pf_gemm_ws_body (N 28672, K 4096, 1021 tokens: 247 against 238 us), which
+// that type keeps.  The eight-wave form of these types, whose loads waited
+// where they were issued (their 2-byte aligned fields were joined at once),
+// took 377 us where this takes 124 (Q6_K, N 3072, K 8192, 1021 tokens), 58
+// against 50 (Q8_0, N 8960, K 1536) and 125 against 69 (F16, N 4096, K 4096).
+template <int FMT, int EPI, bool HALF>
+__device__ __attribute__((always_inline)) void pf_gemm_wr_tile(const PfGemmArgs &a, _Float16 *xs0, _Float16 *xs1, _Float16 *ws0,
+                                                               _Float16 *ws1, uint32_t m0, uint32_t n0) {
+    constexpr int MI = HALF ? 2 : 4;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t nk = a.K / PG_BK;
+    if (wave < 8) {
+        const uint32_t wm = HALF ? 64 * (wave & 3u) : 128 * (wave & 1u), wn = HALF ? 64 * (wave >> 2) : 64 * (wave >> 1);
+        const uint32_t li = lane & 31u, hi = lane >> 5;
+        const _Float16 *x = (const _Float16 *)a.x;
+        uint32_t xoff[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t row = 32 * wave + 8 * (uint32_t)j + (lane >> 3);
+            xoff[j] = 2 * (min(m0 + row, a.M - 1) * a.ldx + 8 * ((lane & 7u) ^ pg_swz_of(row)));
+        }
+        const uint32_t xdst0 = lds_addr(xs0 + (32 * wave) * PG_BK), xdst1 = lds_addr(xs1 + (32 * wave) * PG_BK);
+        auto load_x = [&](uint32_t dst, uint32_t s) {
+            const uint32_t k = min(s, nk - 1) * PG_BK;
+#pragma unroll
+            for (int j = 0; j < 4; j++) lds_dma16(x + k, xoff[j], __builtin_amdgcn_readfirstlane(dst + 1024 * j));
+        };
+        float16v acc[MI][2];
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+        auto products = [&](const _Float16 *xb, const _Float16 *wb) {
+#pragma unroll
+            for (int kk = 0; kk < 4; kk++) {
+                half8v av[MI], bv[2];
+                const uint32_t c = 2 * (uint32_t)kk + hi;
+#pragma unroll
+                for (int i = 0; i < MI; i++) av[i] = *(const half8v *)(xb + pg_swz(wm + 32 * i + li, c));
+#pragma unroll
+                for (int j = 0; j < 2; j++) bv[j] = *(const half8v *)(wb + pg_swz(wn + 32 * j + li, c));
+#pragma unroll
+                for (int i = 0; i < MI; i++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[i], bv[j], acc[i][j], 0, 0, 0);
+            }
+        };
+        load_x(xdst0, 0);
+        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        for (uint32_t s = 0; s < nk; s += 2) {
+            load_x(xdst1, s + 1);
+            products(xs0, ws0);
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (s + 1 < nk) {
+                load_x(xdst0, s + 2);
+                products(xs1, ws1);
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            }
+        }
+        if (EPI == PG_STORE && a.rope)
+            pg_epilogue_rope<MI>(a, acc, lane, wm, wn, m0, n0);
+        else
+            pg_epilogue<EPI, MI>(a, acc, lane, wm, wn, m0, n0);
+        return;
+    }
+    constexpr int NP = HALF ? 1 : 2, D = FMT == F32 ? 1 : 2;
+    const uint32_t t = tid - 512u, r = HALF ? t >> 1 : t, p0 = HALF ? t & 1u : 0u;
+    const uint8_t *wrow = pg_wrow<EPI>(a, n0, r);
+    auto kof = [&](uint32_t s) { return min(s, nk - 1) * PG_BK; };
+    struct Runs {
+        PgRun<FMT> run[NP];
+    } st[D];
+    auto load = [&](Runs &w, uint32_t s) {
+#pragma unroll
+        for (int i = 0; i < NP; i++) w.run[i].load(wrow, kof(s), p0 + (uint32_t)i);
+    };
+    auto put = [&](Runs &w, uint32_t s) {
+        _Float16 *tile = s & 1u ? ws1 : ws0;
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            w.run[i].pin();
+            w.run[i].template store<0>(kof(s), p0 + (uint32_t)i, tile, r, 0);
+            w.run[i].template store<1>(kof(s), p0 + (uint32_t)i, tile, r, 0);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < D; i++) load(st[i], (uint32_t)i);
+    put(st[0], 0);
+    load(st[0], D);
+    lds_barrier();
+    // step s: the weights of step s + 1 into the other buffer, their
+    // registers refilled with step s + 1 + D
+    uint32_t s = 0;
+    for (; s + 2 <= nk; s += 2) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            put(st[(i + 1) % D], s + (uint32_t)i + 1);
+            load(st[(i + 1) % D], s + (uint32_t)i + 1 + D);
+            lds_barrier();
+        }
+    }
+    if (s < nk) {
+        put(st[1 % D], s + 1);
+        lds_barrier();
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70); // the last loads land (vmcnt 0), as in device/pf_small.h
+}
+template <int FMT, int EPI>
+__device__ __attribute__((always_inline)) void pf_gemm_wr_body(const PfGemmArgs &a) {
+    __shared__ __attribute__((aligned(1024))) _Float16 xs0[PG_BM * PG_BK], xs1[PG_BM * PG_BK];
+    __shared__ __attribute__((aligned(1024))) _Float16 ws0[PG_BN * PG_BK], ws1[PG_BN * PG_BK];
+    uint32_t m0, n0;
+    if (pg_tile_ws(a, m0, n0)) // (uniform)
+        pf_gemm_wr_tile<FMT, EPI, true>(a, xs0, xs1, ws0, ws1, m0, n0);
+    else
+        pf_gemm_wr_tile<FMT, EPI, false>(a, xs0, xs1, ws0, ws1, m0, n0);
 }
 
 } // namespace ifr

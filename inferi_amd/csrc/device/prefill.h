@@ -11,150 +11,10 @@
 // which produces the logits and the next token.
 #pragma once
 #include "attention.h"
-#include "pf_gemm.h"
-#include "pf_tiles.h"
+#include "pf_small.h"
 
 namespace ifr {
 
-
-// ------------------------------------------------------------------ GEMM --
-// The small-tile form of the prefill GEMM (device/pf_gemm.h has the
-// 256 x 256 form and the argument conventions): Y[m][n] = sum_k X[m][k] *
-// deq(W)[n][k] with the same epilogues (EPI: PG_STORE, PG_ADD, PG_SWIGLU)
-// and stacked matrices, for products with too few 256 x 256 tiles to fill
-// the chip.  Tile 128 (m) x 128 (n), K steps of 64; four waves, each a
-// 64 x 64 quadrant as 2 x 2 MFMA 32x32x16 tiles.  The next K step's global
-// loads are issued before the current step's MFMAs.  Each output element
-// sums its k in the same order as the large form (steps of 64, products of
-// 16), so both forms give the same results bit for bit.
-constexpr int PF_BM = 128, PF_BN = 128, PF_BK = 64;
-constexpr int PF_LDS = PF_BK + 8; // halves per LDS row: 144 B, so the 32 rows an MFMA operand read touches spread over the banks
-
-template <int FMT, int EPI>
-__device__ void gemm_f16_body(const PfGemmArgs &a) {
-    __shared__ __attribute__((aligned(16))) _Float16 xs[PF_BM][PF_LDS];
-    __shared__ __attribute__((aligned(16))) _Float16 ws[PF_BN][PF_LDS];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t m0 = blockIdx.y * PF_BM, n0 = blockIdx.x * PF_BN;
-
-    // global -> register staging: thread t owns tile row t/2, halves
-    // [32*(t%2), +32); rows past M or N repeat the last row (their outputs
-    // are not stored)
-    const uint32_t r = (uint32_t)tid >> 1, hseg = (uint32_t)tid & 1u;
-    const _Float16 *xrow = (const _Float16 *)a.x + (size_t)min(m0 + r, a.M - 1) * a.ldx;
-    const uint8_t *wrow;
-    if constexpr (EPI == PG_SWIGLU) {
-        // wave column c = r / 64 holds FFN rows j in [n0 / 2 + 32 c, +32):
-        // tile rows 64 c + i are gate row j, 64 c + 32 + i up row j
-        const uint32_t j = min(n0 / 2 + 32 * (r >> 6) + (r & 31u), a.n1 - 1);
-        wrow = ((r >> 5) & 1u ? a.w1 : a.w0) + (size_t)j * a.row_bytes;
-    } else {
-        const uint32_t n = min(n0 + r, a.N - 1);
-        const uint8_t *base = n < a.n1 ? a.w0 : n < a.n2 ? a.w1 : a.w2;
-        const uint32_t nr = n < a.n1 ? n : n < a.n2 ? n - a.n1 : n - a.n2;
-        wrow = base + (size_t)nr * a.row_bytes;
-    }
-    u32x4_a16 x0, x1, x2, x3; // the next K step's X segment
-    PfTile<FMT> wt;
-    float16v acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
-
-    const uint32_t wm = 64 * (uint32_t)(wave >> 1), wn = 64 * (uint32_t)(wave & 1);
-    const uint32_t li = (uint32_t)lane & 31u, lk = 8 * ((uint32_t)lane >> 5);
-    const u32x4_a16 *xp = (const u32x4_a16 *)(xrow + 32 * hseg);
-    x0 = xp[0], x1 = xp[1], x2 = xp[2], x3 = xp[3];
-    wt.load(wrow, 0, hseg);
-    for (uint32_t k0 = 0; k0 < a.K; k0 += PF_BK) {
-        __syncthreads(); // the previous step's operand reads are done
-        {
-            // this thread's 32 weights into LDS as f16, then its X segment
-            _Float16 h[32];
-            wt.deq(k0, hseg, h);
-            uint4 *wd = (uint4 *)&ws[r][32 * hseg];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                uint4 u;
-                __builtin_memcpy(&u, &h[8 * i], 16);
-                wd[i] = u;
-            }
-            u32x4_a16 *xd = (u32x4_a16 *)&xs[r][32 * hseg];
-            xd[0] = x0, xd[1] = x1, xd[2] = x2, xd[3] = x3;
-        }
-        if (k0 + PF_BK < a.K) {
-            const u32x4_a16 *xn = xp + (k0 + PF_BK) / 8;
-            x0 = xn[0], x1 = xn[1], x2 = xn[2], x3 = xn[3];
-            wt.load(wrow, k0 + PF_BK, hseg);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < PF_BK; kk += 16) {
-            half8v av[2], bv[2];
-#pragma unroll
-            for (int i = 0; i < 2; i++) av[i] = *(const half8v *)&xs[wm + 32 * i + li][kk + lk];
-#pragma unroll
-            for (int j = 0; j < 2; j++) bv[j] = *(const half8v *)&ws[wn + 32 * j + li][kk + lk];
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[i], bv[j], acc[i][j], 0, 0, 0);
-        }
-    }
-    // D[row][col]: col = lane % 32, row = 8*(e/4) + 4*(lane/32) + e%4
-    if constexpr (EPI == PG_SWIGLU) {
-        const uint32_t jn = n0 / 2 + wn / 2 + li;
-        if (jn >= a.n1) return;
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) {
-                const uint32_t m = m0 + wm + 32 * i + 8 * (e / 4) + 4 * ((uint32_t)lane >> 5) + (e % 4);
-                if (m < a.M) {
-                    const float g = acc[i][0][e], u = acc[i][1][e];
-                    ((_Float16 *)a.y)[(size_t)m * a.ldy + jn] = f16_of(u * silu_fast(g));
-                }
-            }
-    } else {
-        // eight values at a time; their residual loads (ADD) go out together
-        // from rows clamped below M, so a lane waits once per eight values,
-        // not once per value behind its bounds branch (eight, not sixteen:
-        // the form keeps its three waves per SIMD)
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const uint32_t n = n0 + wn + 32 * j + li;
-                if (n >= a.N) continue;
-#pragma unroll
-                for (int h = 0; h < 16; h += 8) {
-                    float old[8];
-                    if constexpr (EPI == PG_ADD) {
-#pragma unroll
-                        for (int e = h; e < h + 8; e++) {
-                            const uint32_t m = m0 + wm + 32 * i + 8 * (e / 4) + 4 * ((uint32_t)lane >> 5) + (e % 4);
-                            old[e - h] = ((const float *)a.y)[(size_t)min(m, a.M - 1) * a.ldy + n];
-                        }
-                    }
-#pragma unroll
-                    for (int e = h; e < h + 8; e++) {
-                        const uint32_t m = m0 + wm + 32 * i + 8 * (e / 4) + 4 * ((uint32_t)lane >> 5) + (e % 4);
-                        if (m < a.M) {
-                            float *yp = (float *)a.y + (size_t)m * a.ldy + n;
-                            if constexpr (EPI == PG_ADD)
-                                *yp = old[e - h] + acc[i][j][e];
-                            else
-                                *yp = acc[i][j][e];
-                        }
-                    }
-                }
-            }
-    }
-}
 
 // ------------------------------------------------------------ pointwise --
 

@@ -46,7 +46,6 @@ uint64_t xq_bytes(uint64_t n) { return 3 * n + n / 2; }
 constexpr uint32_t ATTN_SPLITS_MAX = 256; // attention splits per KV head (at most)
 constexpr uint32_t ATTN_GT_MAX = 8;       // device/attention.h: query heads per workgroup
 constexpr uint32_t MAX_PARTS = 1024;      // argmax partial keys per launch
-constexpr uint32_t PF_GEMM_TILE = 128;    // device/prefill.h: PF_BM = PF_BN
 constexpr uint32_t PF_BIG_TILE = 256;     // device/pf_gemm.h: PG_BM = PG_BN
 constexpr uint32_t PF_BIG_THREADS = 512;  // device/pf_gemm.h: PG_THREADS
 constexpr uint32_t PF_WS_THREADS = 768;   // device/pf_gemm.h: PGW_THREADS
@@ -140,16 +139,15 @@ struct ifr_ctx {
     uint32_t pf_chunk = 0;
     // this device's fixed scratch of ifr_matmul_quant_noalloc (noalloc.hip)
     void *noalloc_scratch = nullptr;
-    // prefill GEMM tiles: 0 = by shape (256 x 256 tiles where the product
-    // has enough of them, else 128 x 128), 128 or 256 to force one (option
-    // pf_tile)
+    // prefill GEMM tiles: 0 = by shape (pf_small_form), 128 or 256 to force
+    // one (option pf_tile)
     uint32_t pf_tile = 0;
     // Q4_K products on 256 x 256 tiles in the warp-specialized form (option
     // pf_ws, default on; 0 = the eight-wave form; device/pf_gemm.h
     // pf_gemm_ws_body)
     int pf_ws = 1;
     // the Q/K/V product's epilogue applies RoPE and stores k, v to the cache
-    // (warp-specialized form, pairs (2i, 2i + 1)) instead of pf_rope_kv_k
+    // (not in the eight-wave form; pairs (2i, 2i + 1)) instead of pf_rope_kv_k
     // (option pf_rope_fuse, default on)
     int pf_rope_fuse = 1;
     // bumped by every option change: a captured decode step is captured
@@ -1702,24 +1700,45 @@ static ifr_status check_weights(ifr_ctx *c, const ifr_llama2_state *s, const ifr
 
 // Y[m][n] (+)= sum_k Xh[m][k] * deq(W)[n][k] on the matrix cores, the weight
 // tiles dequantized to f16 inside the kernels (device/pf_gemm.h: 256 x 256
-// tiles; device/prefill.h gemm_f16_body: 128 x 128 tiles, the same results
-// bit for bit).
+// tiles; device/pf_small.h: smaller ones, the same results bit for bit).
 static uint32_t pf_row_bytes(const Tens &w) {
     return (w.cols / (uint32_t)qk_of(w.dtype)) * (uint32_t)bytes_of(w.dtype);
 }
 
 enum PfEpi { PF_EPI_STORE = 0, PF_EPI_ADD = 1, PF_EPI_SWIGLU = 2 };
-// Products with at least this many 256 x 256 tiles take that form (every
-// product of a 4096-token pass at the 8B shape: 256 to 1792 tiles); smaller
-// ones run 128 x 128 tiles, four times the workgroups.
-constexpr uint32_t PF_BIG_TILES_MIN = 128;
+// The small-tile forms (device/pf_small.h).
+struct PfSmallForm {
+    uint32_t bm, bn, threads;
+    const char *name;
+};
+constexpr PfSmallForm PF_T32{32, 32, 6 * 64, "_t32_"}, PF_T64{64, 64, 7 * 64, "_t64_"}, PF_T128{128, 128, 8 * 64, "_t128_"};
+// The smallest tile whose grid the chip takes at once, null for the 256 x 256
+// form: 32 x 32 while its tiles are no more than the CUs, 64 x 64 to two per
+// CU, 128 x 128 to one (a wider tile re-reads and stages less per product,
+// but leaves CUs idle below that).  Both sides of each line, us per product,
+// Q4_K unless said: 32 x 32 against 64 x 64 at 256 tiles (N 4096, K 14336, 61
+// tokens) 37 against 64, at 384 (N 6144, K 4096, 61) 22.4 against 21.5; 64
+// against 128 at 512 (N 4096, K 14336, 512) 128 against 140, at 560 (Q8_0, N
+// 8960, K 1536, 256) 27.4 against 24.5; 128 against 256 at 256 (N 4096, K
+// 4096, 1021) 56 against 66, at 280 (Q8_0, N 8960, K 1536, 509) 43 against
+// 31.  A tile twice as high as the tokens only pads: up to 64 and 128 tokens
+// the larger forms are not taken (N 28672, K 4096: 61 tokens 39 with 64 x 64,
+// 52 with 128 x 128; 128 tokens 52 with 128 x 128, 78 with 256 x 256).  The
+// SwiGLU epilogue needs the 64 columns of a gate and an up block.
+static const PfSmallForm *pf_small_form(uint32_t n_cu, uint32_t M, uint32_t N, PfEpi epi) {
+    auto tiles = [&](uint32_t t) { return (uint64_t)((M + t - 1) / t) * ((N + t - 1) / t); };
+    if (epi != PF_EPI_SWIGLU && tiles(32) <= n_cu) return &PF_T32;
+    if (M <= 64 || tiles(64) <= 2 * (uint64_t)n_cu) return &PF_T64;
+    if (M <= 128 || tiles(128) <= n_cu) return &PF_T128;
+    return nullptr;
+}
 
 // One product of a pass: nm (1 to 3) matrices of one type stacked by rows
 // into Y[M][ldy] f32 (stored or added), or (SwiGLU) gate m[0] and up m[1]
 // into h[M][ldy] = f16(up * silu(gate)).  X rows (pitch ldx halves) must be
 // 16-byte aligned.  rope (may be null): the stacked Q | K | V store product
-// may fuse pf_rope_kv_k's work into its epilogue (warp-specialized form
-// only); *fused says whether it did.
+// may fuse pf_rope_kv_k's work into its epilogue (not in the eight-wave
+// form); *fused says whether it did.
 static ifr_status launch_pf_gemm(ifr_ctx *c, const void *xh, uint32_t ldx, const Tens *const *m, int nm, void *y,
                                  uint32_t ldy, uint32_t M, PfEpi epi, const PfArgs *rope = nullptr,
                                  bool *fused = nullptr) {
@@ -1748,33 +1767,52 @@ static ifr_status launch_pf_gemm(ifr_ctx *c, const void *xh, uint32_t ldx, const
     static const char *epi_name[3] = {"store", "add", "swiglu"};
     // the large form addresses X rows with 32-bit byte offsets
     const bool big_ok = (uint64_t)M * ldx * 2 < (1ull << 32);
-    const bool big = big_ok && (c->pf_tile == 256 || (c->pf_tile == 0 && g.tiles_n * g.tiles_m >= PF_BIG_TILES_MIN));
-    if (big && c->pf_ws && m[0]->dtype == IFR_Q4_K) {
+    const PfSmallForm *small = c->pf_tile == 128 ? &PF_T128 : c->pf_tile == 256 ? nullptr : pf_small_form((uint32_t)c->n_cu, M, g.N, epi);
+    const bool big = big_ok && !small;
+    if (!small) small = &PF_T128;
+    // fuse RoPE and the KV store into a stacked Q | K | V product
+    auto fuse_rope = [&]() {
+        if (!rope || epi != PF_EPI_STORE || nm != 3) return;
+        g.rope = 1;
+        g.rope_cs = rope->rope_cs;
+        g.q_bias = rope->q_bias;
+        g.k_bias = rope->k_bias;
+        g.v_bias = rope->v_bias;
+        g.k_cache = rope->k_cache;
+        g.v_cache = rope->v_cache;
+        g.head_size = rope->head_size;
+        g.p0 = rope->p0;
+        g.kv_f16 = rope->kv_f16;
+        if (fused) *fused = true;
+    };
+    if (big && (c->pf_ws || m[0]->dtype != IFR_Q4_K)) {
         // a last round of at most 128 tiles (half the CUs) runs as twice as
         // many 256 x 128 halves, one round over every CU
         const uint32_t tiles = g.tiles_n * g.tiles_m, tail = tiles % PF_WS_ROUND;
         g.tiles_full = tail != 0 && tail <= PF_WS_ROUND / 2 ? tiles - tail : tiles;
-        if (rope && epi == PF_EPI_STORE && nm == 3) {
-            g.rope = 1;
-            g.rope_cs = rope->rope_cs;
-            g.q_bias = rope->q_bias;
-            g.k_bias = rope->k_bias;
-            g.v_bias = rope->v_bias;
-            g.k_cache = rope->k_cache;
-            g.v_cache = rope->v_cache;
-            g.head_size = rope->head_size;
-            g.p0 = rope->p0;
-            g.kv_f16 = rope->kv_f16;
-            if (fused) *fused = true;
-        }
-        return c->launch(std::string("pf_gemm_q4_k_ws_") + epi_name[epi], dim3(tiles + (tiles - g.tiles_full)),
-                         dim3(PF_WS_THREADS), 0, g);
+        fuse_rope();
+        return c->launch(std::string("pf_gemm_") + gemv_fmt_name(m[0]->dtype) + "_ws_" + epi_name[epi],
+                         dim3(tiles + (tiles - g.tiles_full)), dim3(PF_WS_THREADS), 0, g);
     }
     if (big)
-        return c->launch(std::string("pf_gemm_") + gemv_fmt_name(m[0]->dtype) + "_" + epi_name[epi],
-                         dim3(g.tiles_n * g.tiles_m), dim3(PF_BIG_THREADS), 0, g);
-    const dim3 grid((g.N + PF_GEMM_TILE - 1) / PF_GEMM_TILE, (M + PF_GEMM_TILE - 1) / PF_GEMM_TILE);
-    return c->launch(std::string("gemm_") + gemv_fmt_name(m[0]->dtype) + "_f16_" + epi_name[epi], grid, dim3(256), 0, g);
+        return c->launch(std::string("pf_gemm_q4_k_") + epi_name[epi], dim3(g.tiles_n * g.tiles_m), dim3(PF_BIG_THREADS), 0, g);
+    const PfSmallForm &f = *small;
+    g.tiles_n = (g.N + f.bn - 1) / f.bn;
+    const std::string name = std::string("pf_gemm_") + gemv_fmt_name(m[0]->dtype) + f.name + epi_name[epi];
+    // a tile addresses its X rows with 32-bit byte offsets from its first
+    // one: rows so long that a tile's offsets do not fit go a few at a time
+    const uint64_t row = (uint64_t)ldx * 2;
+    const uint32_t per = row * f.bm < (1ull << 32) ? M : (uint32_t)std::max<uint64_t>(1, ((1ull << 32) - 1) / row);
+    if (per >= M) fuse_rope();
+    for (uint32_t r0 = 0; r0 < M; r0 += per) {
+        g.M = std::min(per, M - r0);
+        g.tiles_m = (g.M + f.bm - 1) / f.bm;
+        g.x = (const uint8_t *)xh + r0 * row;
+        g.y = (uint8_t *)y + (uint64_t)r0 * ldy * (epi == PF_EPI_SWIGLU ? 2 : 4);
+        ifr_status st = c->launch(name, dim3(g.tiles_n * g.tiles_m), dim3(f.threads), 0, g);
+        if (st) return st;
+    }
+    return IFR_OK;
 }
 
 // A matrix the prefill GEMM takes: a quantized GGUF type, K a whole number

@@ -44,20 +44,23 @@ using namespace ifr;
     extern "C" __global__ void __launch_bounds__(RW * KS * 64) NAME##_r##R##w##RW##k##KS(GemvArgs a) { \
         gemv_grp_body<FMT, MODE, R, RW, KS>(a);                                                         \
     }
-// gate/up with h in f32, and the down GEMV that quantizes its f32 input itself
-extern "C" __global__ void __launch_bounds__(GEMV_ONE_WAVES * 64) gemv_q4_k_gateup_one(GemvArgs a) {
-    gemv_one_body<Q4_K, GEMV_GATEUP>(a);
-}
-// one-item forms with four rows per wave (option gemv_grp bits 7 and 8)
+
+// The kernels of the usual decode step (Q4_K layers, Q6_K head), in the order
+// it runs them and next to each other: together they are 43 KB, which the
+// instruction caches (64 KB per two CUs) hold from one step to the next if
+// they do not fall on the same sets.  Wherever the rest of the code object
+// had put them before, the same step took 493.5 to 499.5 us on the 8B widths
+// with eight layers (as other kernels were added), here 493.
+extern "C" __global__ void __launch_bounds__(256) embed_k(EmbedArgs a) { embed_body(a); }
+GEMV_ONE_KERNEL(gemv_q4_k_qkv, Q4_K, GEMV_QKV)
+extern "C" __global__ void __launch_bounds__(256) attn_f16_h128_g4(AttnArgs a) { attn_split_body<128, 4, true>(a); }
+extern "C" __global__ void __launch_bounds__(64) attn_merge(AttnArgs a) { attn_merge_body(a); }
+GEMV_GRP_KERNEL(gemv_q4_k_resid, Q4_K, GEMV_RESID, 2, 8, 1)
+// gate/up with h in f32, four rows per wave (option gemv_grp bit 7)
 extern "C" __global__ void __launch_bounds__(GEMV_ONE_WAVES * 64) gemv_q4_k_gateup_one4(GemvArgs a) {
     gemv_one_body<Q4_K, GEMV_GATEUP, 4>(a);
 }
-extern "C" __global__ void __launch_bounds__(GEMV_ONE_WAVES * 64) gemv_q4_k_qkv_one4(GemvArgs a) {
-    gemv_one_body<Q4_K, GEMV_QKV, 4>(a);
-}
-extern "C" __global__ void __launch_bounds__(GEMV_ONE_WAVES * 64) gemv_q4_k_plain_one4(GemvArgs a) {
-    gemv_one_body<Q4_K, GEMV_PLAIN, 4>(a);
-}
+// the down GEMV that quantizes its f32 input itself
 extern "C" __global__ void __launch_bounds__(GEMV_INT_MAX_WAVES * 64)
     __attribute__((amdgpu_waves_per_eu(GEMV_INT_WPE, 8))) gemv_q4_k_resid_xf(GemvArgs a) {
     gemv_int_body<Q4_K, GEMV_RESID, GEMV_INT_PIPE, GEMV_INT_NI, true>(a);
@@ -68,7 +71,19 @@ extern "C" __global__ void __launch_bounds__(4 * 64) __attribute__((amdgpu_waves
 gemv_q6_k_head_w2(GemvArgs a) {
     gemv_int_body<Q6_K, GEMV_HEAD, GEMV_INT_PIPE, GEMV_INT_NI>(a);
 }
-GEMV_GRP_KERNEL(gemv_q4_k_resid, Q4_K, GEMV_RESID, 2, 8, 1)
+extern "C" __global__ void __launch_bounds__(1024) argmax_final_k(ArgmaxArgs a) { argmax_final_body(a); }
+
+// gate/up with h in f32, two rows per wave
+extern "C" __global__ void __launch_bounds__(GEMV_ONE_WAVES * 64) gemv_q4_k_gateup_one(GemvArgs a) {
+    gemv_one_body<Q4_K, GEMV_GATEUP>(a);
+}
+// one-item forms with four rows per wave (option gemv_grp bit 8)
+extern "C" __global__ void __launch_bounds__(GEMV_ONE_WAVES * 64) gemv_q4_k_qkv_one4(GemvArgs a) {
+    gemv_one_body<Q4_K, GEMV_QKV, 4>(a);
+}
+extern "C" __global__ void __launch_bounds__(GEMV_ONE_WAVES * 64) gemv_q4_k_plain_one4(GemvArgs a) {
+    gemv_one_body<Q4_K, GEMV_PLAIN, 4>(a);
+}
 GEMV_GRP_KERNEL(gemv_q4_k_resid, Q4_K, GEMV_RESID, 4, 4, 4)
 GEMV_GRP_KERNEL(gemv_q4_k_gateup, Q4_K, GEMV_GATEUP, 4, 8, 1)
 GEMV_GRP_KERNEL(gemv_q4_k_gateup, Q4_K, GEMV_GATEUP, 2, 16, 1)
@@ -90,7 +105,6 @@ GEMV_GRP_KERNEL(gemv_q4_k_gateup, Q4_K, GEMV_GATEUP, 2, 16, 1)
     GEMV_ONE_KERNEL(gemv_##FMTNAME##_plain, FMT, GEMV_PLAIN) \
     GEMV_ONE_XF_KERNEL(gemv_##FMTNAME##_plain, FMT)          \
     GEMV_XF_KERNEL(gemv_##FMTNAME##_plain, FMT)              \
-    GEMV_ONE_KERNEL(gemv_##FMTNAME##_qkv, FMT, GEMV_QKV)     \
     GEMV_ONE_KERNEL(gemv_##FMTNAME##_head, FMT, GEMV_HEAD)   \
     GEMV_KERNEL(gemv_##FMTNAME##_plain, FMT, GEMV_PLAIN)   \
     GEMV_KERNEL(gemv_##FMTNAME##_resid, FMT, GEMV_RESID)   \
@@ -99,73 +113,107 @@ GEMV_GRP_KERNEL(gemv_q4_k_gateup, Q4_K, GEMV_GATEUP, 2, 16, 1)
     GEMV_KERNEL(gemv_##FMTNAME##_head, FMT, GEMV_HEAD)
 
 GEMV_ALL_MODES(q4_k, Q4_K)
+GEMV_ONE_KERNEL(gemv_q5_k_qkv, Q5_K, GEMV_QKV)
 GEMV_ALL_MODES(q5_k, Q5_K)
+GEMV_ONE_KERNEL(gemv_q6_k_qkv, Q6_K, GEMV_QKV)
 GEMV_ALL_MODES(q6_k, Q6_K)
+GEMV_ONE_KERNEL(gemv_q8_0_qkv, Q8_0, GEMV_QKV)
 GEMV_ALL_MODES(q8_0, Q8_0)
+GEMV_ONE_KERNEL(gemv_q4_0_qkv, Q4_0, GEMV_QKV)
 GEMV_ALL_MODES(q4_0, Q4_0)
+GEMV_ONE_KERNEL(gemv_q4_1_qkv, Q4_1, GEMV_QKV)
 GEMV_ALL_MODES(q4_1, Q4_1)
+GEMV_ONE_KERNEL(gemv_q5_0_qkv, Q5_0, GEMV_QKV)
 GEMV_ALL_MODES(q5_0, Q5_0)
+GEMV_ONE_KERNEL(gemv_q5_1_qkv, Q5_1, GEMV_QKV)
 GEMV_ALL_MODES(q5_1, Q5_1)
+GEMV_ONE_KERNEL(gemv_q8_k_qkv, Q8_K, GEMV_QKV)
 GEMV_ALL_MODES(q8_k, Q8_K)
+GEMV_ONE_KERNEL(gemv_f16_qkv, F16, GEMV_QKV)
 GEMV_ALL_MODES(f16, F16)
+GEMV_ONE_KERNEL(gemv_f32_qkv, F32, GEMV_QKV)
 GEMV_ALL_MODES(f32, F32)
 
 // decode attention: head sizes padded to 64 or 128, 1..8 query heads per workgroup
-#define ATTN_KERNEL(HSP, GT)                                                                        \
-    extern "C" __global__ void __launch_bounds__(256) attn_f16_h##HSP##_g##GT(AttnArgs a) {         \
-        attn_split_body<HSP, GT, true>(a);                                                          \
-    }                                                                                               \
-    extern "C" __global__ void __launch_bounds__(256) attn_f32_h##HSP##_g##GT(AttnArgs a) {         \
-        attn_split_body<HSP, GT, false>(a);                                                         \
+#define ATTN_KERNEL(HSP, GT, NAME, KV16)                                            \
+    extern "C" __global__ void __launch_bounds__(256) attn_##NAME##_h##HSP##_g##GT(AttnArgs a) { \
+        attn_split_body<HSP, GT, KV16>(a);                                            \
     }
-#define ATTN_KERNELS(HSP) \
-    ATTN_KERNEL(HSP, 1) ATTN_KERNEL(HSP, 2) ATTN_KERNEL(HSP, 3) ATTN_KERNEL(HSP, 4) \
-    ATTN_KERNEL(HSP, 5) ATTN_KERNEL(HSP, 6) ATTN_KERNEL(HSP, 7) ATTN_KERNEL(HSP, 8)
-ATTN_KERNELS(64)
-ATTN_KERNELS(128)
-extern "C" __global__ void __launch_bounds__(64) attn_merge(AttnArgs a) { attn_merge_body(a); }
+#define ATTN_KERNELS(HSP, NAME, KV16)                                                                 \
+    ATTN_KERNEL(HSP, 1, NAME, KV16) ATTN_KERNEL(HSP, 2, NAME, KV16) ATTN_KERNEL(HSP, 3, NAME, KV16) \
+    ATTN_KERNEL(HSP, 5, NAME, KV16) ATTN_KERNEL(HSP, 6, NAME, KV16) ATTN_KERNEL(HSP, 7, NAME, KV16) \
+    ATTN_KERNEL(HSP, 8, NAME, KV16)
+ATTN_KERNELS(64, f16, true)
+ATTN_KERNEL(64, 4, f16, true)
+ATTN_KERNELS(64, f32, false)
+ATTN_KERNEL(64, 4, f32, false)
+ATTN_KERNELS(128, f16, true)
+ATTN_KERNELS(128, f32, false)
+ATTN_KERNEL(128, 4, f32, false)
 
 extern "C" __global__ void __launch_bounds__(1024) rms_norm_k(EltArgs a) { rms_norm_body(a); }
 extern "C" __global__ void __launch_bounds__(256) rope_k(EltArgs a) { rope_body(a); }
 extern "C" __global__ void __launch_bounds__(256) silu_k(EltArgs a) { silu_body(a); }
 extern "C" __global__ void __launch_bounds__(256) add_k(EltArgs a) { add_body(a); }
 extern "C" __global__ void __launch_bounds__(256) argmax_part_k(ArgmaxArgs a) { argmax_part_body(a); }
-extern "C" __global__ void __launch_bounds__(1024) argmax_final_k(ArgmaxArgs a) { argmax_final_body(a); }
 extern "C" __global__ void __launch_bounds__(256) sample_exp_k(SampleArgs a) { sample_exp_body(a); }
 extern "C" __global__ void __launch_bounds__(256) sample_prob_k(SampleArgs a) { sample_prob_body(a); }
 extern "C" __global__ void __launch_bounds__(256) sample_group_k(SampleArgs a) { sample_group_body(a); }
 extern "C" __global__ void __launch_bounds__(1024) sample_select_k(SampleArgs a) { sample_select_body(a); }
-extern "C" __global__ void __launch_bounds__(256) embed_k(EmbedArgs a) { embed_body(a); }
 extern "C" __global__ void __launch_bounds__(256) quant_act_k(QActArgs a) { quant_act_body(a); }
 extern "C" __global__ void __launch_bounds__(256) kv_store_k(KvStoreArgs a) { kv_store_body(a); }
 extern "C" __global__ void __launch_bounds__(256) dequant_k(DequantArgs a) { dequant_body(a); }
 extern "C" __global__ void __launch_bounds__(64) quantize_k(QuantArgs a) { quantize_body(a); }
 extern "C" __global__ void __launch_bounds__(256) fill_normal_k(FillArgs a) { fill_normal_body(a); }
 
-// prompt (prefill) path: the GEMM in 256 x 256 tiles (eight waves, two per
-// SIMD) and in 128 x 128 tiles, each with the store, accumulate and SwiGLU
-// epilogues
-#define PF_GEMM_KERNELS(FMTNAME, FMT)                                                                             \
-    extern "C" __global__ void __launch_bounds__(PG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))           \
-    pf_gemm_##FMTNAME##_store(PfGemmArgs a) {                                                                     \
-        pf_gemm_body<FMT, PG_STORE>(a);                                                                           \
-    }                                                                                                             \
-    extern "C" __global__ void __launch_bounds__(PG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))           \
-    pf_gemm_##FMTNAME##_add(PfGemmArgs a) {                                                                       \
-        pf_gemm_body<FMT, PG_ADD>(a);                                                                             \
-    }                                                                                                             \
-    extern "C" __global__ void __launch_bounds__(PG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))           \
-    pf_gemm_##FMTNAME##_swiglu(PfGemmArgs a) {                                                                    \
-        pf_gemm_body<FMT, PG_SWIGLU>(a);                                                                          \
-    }                                                                                                             \
-    extern "C" __global__ void __launch_bounds__(256) gemm_##FMTNAME##_f16_store(PfGemmArgs a) {                  \
-        gemm_f16_body<FMT, PG_STORE>(a);                                                                          \
-    }                                                                                                             \
-    extern "C" __global__ void __launch_bounds__(256) gemm_##FMTNAME##_f16_add(PfGemmArgs a) {                    \
-        gemm_f16_body<FMT, PG_ADD>(a);                                                                            \
-    }                                                                                                             \
-    extern "C" __global__ void __launch_bounds__(256) gemm_##FMTNAME##_f16_swiglu(PfGemmArgs a) {                 \
-        gemm_f16_body<FMT, PG_SWIGLU>(a);                                                                         \
+// prompt (prefill) path: the GEMM in 32 x 32, 64 x 64 and 128 x 128 tiles and
+// in 256 x 256 tiles (warp-specialized: 12 waves, three per SIMD), each with
+// the store, accumulate and SwiGLU epilogues
+#define PF_GEMM_KERNELS(FMTNAME, FMT)                                                                                 \
+    extern "C" __global__ void __launch_bounds__(PG_T32_THREADS)                                                      \
+    pf_gemm_##FMTNAME##_t32_store(PfGemmArgs a) {                                                                     \
+        pf_gemm_t32_body<FMT, PG_STORE>(a);                                                                           \
+    }                                                                                                                 \
+    extern "C" __global__ void __launch_bounds__(PG_T32_THREADS)                                                      \
+    pf_gemm_##FMTNAME##_t32_add(PfGemmArgs a) {                                                                       \
+        pf_gemm_t32_body<FMT, PG_ADD>(a);                                                                             \
+    }                                                                                                                 \
+    extern "C" __global__ void __launch_bounds__(PG_T64_THREADS)                                                      \
+    pf_gemm_##FMTNAME##_t64_store(PfGemmArgs a) {                                                                     \
+        pf_gemm_t64_body<FMT, PG_STORE>(a);                                                                           \
+    }                                                                                                                 \
+    extern "C" __global__ void __launch_bounds__(PG_T64_THREADS)                                                      \
+    pf_gemm_##FMTNAME##_t64_add(PfGemmArgs a) {                                                                       \
+        pf_gemm_t64_body<FMT, PG_ADD>(a);                                                                             \
+    }                                                                                                                 \
+    extern "C" __global__ void __launch_bounds__(PG_T64_THREADS)                                                      \
+    pf_gemm_##FMTNAME##_t64_swiglu(PfGemmArgs a) {                                                                    \
+        pf_gemm_t64_body<FMT, PG_SWIGLU>(a);                                                                          \
+    }                                                                                                                 \
+    extern "C" __global__ void __launch_bounds__(PG_T128_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4)))          \
+    pf_gemm_##FMTNAME##_t128_store(PfGemmArgs a) {                                                                    \
+        pf_gemm_t128_body<FMT, PG_STORE>(a);                                                                          \
+    }                                                                                                                 \
+    extern "C" __global__ void __launch_bounds__(PG_T128_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4)))          \
+    pf_gemm_##FMTNAME##_t128_add(PfGemmArgs a) {                                                                      \
+        pf_gemm_t128_body<FMT, PG_ADD>(a);                                                                            \
+    }                                                                                                                 \
+    extern "C" __global__ void __launch_bounds__(PG_T128_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4)))          \
+    pf_gemm_##FMTNAME##_t128_swiglu(PfGemmArgs a) {                                                                   \
+        pf_gemm_t128_body<FMT, PG_SWIGLU>(a);                                                                         \
+    }
+#define PF_GEMM_WS_KERNELS(FMTNAME, FMT)                                                                              \
+    extern "C" __global__ void __launch_bounds__(PGW_THREADS)                                                         \
+    pf_gemm_##FMTNAME##_ws_store(PfGemmArgs a) {                                                                      \
+        pf_gemm_wr_body<FMT, PG_STORE>(a);                                                                            \
+    }                                                                                                                 \
+    extern "C" __global__ void __launch_bounds__(PGW_THREADS)                                                         \
+    pf_gemm_##FMTNAME##_ws_add(PfGemmArgs a) {                                                                        \
+        pf_gemm_wr_body<FMT, PG_ADD>(a);                                                                              \
+    }                                                                                                                 \
+    extern "C" __global__ void __launch_bounds__(PGW_THREADS)                                                         \
+    pf_gemm_##FMTNAME##_ws_swiglu(PfGemmArgs a) {                                                                     \
+        pf_gemm_wr_body<FMT, PG_SWIGLU>(a);                                                                           \
     }
 PF_GEMM_KERNELS(q4_k, Q4_K)
 PF_GEMM_KERNELS(q5_k, Q5_K)
@@ -178,7 +226,18 @@ PF_GEMM_KERNELS(q5_0, Q5_0)
 PF_GEMM_KERNELS(q5_1, Q5_1)
 PF_GEMM_KERNELS(f16, F16)
 PF_GEMM_KERNELS(f32, F32)
-// the warp-specialized Q4_K product (option pf_ws): 12 waves, three per SIMD
+PF_GEMM_WS_KERNELS(q5_k, Q5_K)
+PF_GEMM_WS_KERNELS(q6_k, Q6_K)
+PF_GEMM_WS_KERNELS(q8_k, Q8_K)
+PF_GEMM_WS_KERNELS(q8_0, Q8_0)
+PF_GEMM_WS_KERNELS(q4_0, Q4_0)
+PF_GEMM_WS_KERNELS(q4_1, Q4_1)
+PF_GEMM_WS_KERNELS(q5_0, Q5_0)
+PF_GEMM_WS_KERNELS(q5_1, Q5_1)
+PF_GEMM_WS_KERNELS(f16, F16)
+PF_GEMM_WS_KERNELS(f32, F32)
+// Q4_K's own forms on 256 x 256 tiles: warp-specialized, and eight waves that
+// each load, dequantize and multiply (option pf_ws = 0)
 extern "C" __global__ void __launch_bounds__(PGW_THREADS) pf_gemm_q4_k_ws_store(PfGemmArgs a) {
     pf_gemm_ws_body<PG_STORE>(a);
 }
@@ -187,6 +246,15 @@ extern "C" __global__ void __launch_bounds__(PGW_THREADS) pf_gemm_q4_k_ws_add(Pf
 }
 extern "C" __global__ void __launch_bounds__(PGW_THREADS) pf_gemm_q4_k_ws_swiglu(PfGemmArgs a) {
     pf_gemm_ws_body<PG_SWIGLU>(a);
+}
+extern "C" __global__ void __launch_bounds__(PG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) pf_gemm_q4_k_store(PfGemmArgs a) {
+    pf_gemm_body<PG_STORE>(a);
+}
+extern "C" __global__ void __launch_bounds__(PG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) pf_gemm_q4_k_add(PfGemmArgs a) {
+    pf_gemm_body<PG_ADD>(a);
+}
+extern "C" __global__ void __launch_bounds__(PG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) pf_gemm_q4_k_swiglu(PfGemmArgs a) {
+    pf_gemm_body<PG_SWIGLU>(a);
 }
 extern "C" __global__ void __launch_bounds__(256) pf_embed_k(PfArgs a) { pf_embed_body(a); }
 extern "C" __global__ void __launch_bounds__(256) pf_rmsnorm_f16_k(PfArgs a) { pf_rmsnorm_f16_body(a); }

@@ -409,3 +409,67 @@ def test_prefill_rejects_unsupported(ctx):
         w.close()
         s.close()
         w.close()
+
+
+# products whose grid picks each tile form by itself, at its edges: 32 x 32
+# (one row and column of tiles, ragged ones, 256 tiles), 64 x 64 (257 of the
+# former; tokens up to 64 with any width), 128 x 128 and 256 x 256; K of whole
+# and of partial 128- and 256-wide steps
+AUTO = [(32, 256, 1), (33, 512, 31), (1000, 1280, 33), (4096, 256, 64), (4097, 256, 64), (16500, 256, 64),
+        (4160, 512, 300), (1030, 768, 2000), (4500, 256, 1100)]
+AUTO_SHORT_K = [(40, 64, 5), (96, 192, 70), (900, 896, 129), (5000, 320, 200)]
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+def test_gemm_quant_tile_by_shape(ctx, fmt):
+    """The form a product takes by its shape (pf_tile 0) against the forced
+    256 x 256 form (held to the f64 product above): the same bits, stored and
+    accumulated."""
+    import inferi_amd as I
+
+    dtype = getattr(I, fmt)
+    rng = np.random.default_rng(dtype)
+    for rows, cols, m in AUTO + (AUTO_SHORT_K if I.BLOCK_ELEMS[dtype] < 256 else []):
+        w = synthetic_q(ctx, rows, cols, rows + cols, dtype)
+        dx = ctx.upload(rng.standard_normal((m, cols)).astype(np.float16))
+        y = ctx.alloc(m * rows * 4)
+        out = {}
+        for tile in (0, 256):
+            ctx.set_option("pf_tile", tile)
+            try:
+                ctx.gemm_quant(y, w, dtype, rows, cols, dx, m)
+                a = y.download(np.uint32, m * rows)
+                ctx.gemm_quant(y, w, dtype, rows, cols, dx, m, accumulate=True)
+                out[tile] = (a, y.download(np.uint32, m * rows))
+            finally:
+                ctx.set_option("pf_tile", 0)
+        for a, b in zip(out[0], out[256]):
+            assert np.array_equal(a, b), f"{rows}x{cols}, {m} tokens"
+        for b in (w, dx, y):
+            b.free()
+
+
+@pytest.mark.parametrize("mat,kv,bias,n", [("Q8_0", "F32", True, 9), ("Q4_K", "F16", False, 61), ("Q5_0", "F16", True, 150),
+                                           ("Q6_K", "F32", False, 700), ("F16", "F16", False, 1100)])
+def test_prefill_short_prompt_forms(ctx, mat, kv, bias, n):
+    """Prompts whose products take the small tiles: RoPE and the KV store in
+    the Q/K/V epilogue or in a kernel of their own, and forced 256 x 256
+    tiles, give the same KV rows, logits and tokens bit for bit."""
+    import inferi_amd as I
+
+    cfg = I.Llama2Config(n_layers=3, hidden=768, ffn=1536, n_heads=12, n_kv_heads=4, vocab=500, max_pos=1200,
+                         rope_theta=10000.0, rms_eps=1e-5, kv_dtype=getattr(I, kv))
+    w = I.Llama2Weights.synthetic(ctx, cfg, seed=n, mat_dtype=getattr(I, mat), std=0.05, qkv_bias=bias)
+    prompt = np.random.default_rng(n).integers(0, cfg.vocab, n + 1).astype(np.uint32)
+    out = {}
+    try:
+        for tile, fuse in ((0, 1), (0, 0), (256, 0)):
+            ctx.set_option("pf_tile", tile)
+            ctx.set_option("pf_rope_fuse", fuse)
+            out[tile, fuse] = _prefill_run(ctx, cfg, w, prompt, n, 3)
+    finally:
+        ctx.set_option("pf_tile", 0)
+        ctx.set_option("pf_rope_fuse", 1)
+        w.close()
+    for key in ((0, 0), (256, 0)):
+        _same(out[0, 1], out[key], f"tile {key[0]}, fuse {key[1]}")
