@@ -1,12 +1,14 @@
-// Flash-decoding attention for one token over a [seq][kv_dim] KV cache.
+// Flash-decoding attention for one token over a [seq][kv_dim] KV cache: split
+// over the sequence with a merge (below), or for short contexts in one kernel
+// (attn_one_body, at the end).
 //
 // Grid (n_kv_heads * n_sub, n_splits).  Workgroup (x, s) serves up to GT of
 // the G = kv_mul query heads that share KV head h = x / n_sub: heads
 // (x % n_sub) * GT .. +GT of the group, those below G (grouped-query
 // attention reads each K/V row once for all of them, where the reference's
 // fused_attention reads it once per query head: fused_attention.rs:66-241,
-// which takes any kv_mul and head size).  A group of more than 8 heads is
-// split into n_sub sub-groups of GT.  Workgroup (x, s) covers the s-th chunk
+// which takes any kv_mul and head size).  A larger group is split into n_sub
+// sub-groups of GT.  Workgroup (x, s) covers the s-th chunk
 // of the positions [0, pos].  The chunk length is ceil((pos+1)/n_splits)
 // rounded up to whole batches, computed on the device from the
 // device-resident position, so one launch shape serves every position (and a
@@ -419,6 +421,144 @@ __device__ inline void attn_merge_body(const AttnArgs &a) {
     const bool ok = lane < 16 && in;
     if (ok && a.out) a.out[oi] = res;
     if (a.xq_out) quant16(ok ? res : 0.0f, ok, a.xq_out, a.n_out, oi, lane);
+}
+
+// ------------------------------------------------ attention in one kernel --
+// Short contexts: one workgroup per query head takes every position, so
+// there are no partials and no merge launch.  Grid n_heads; blockDim 64 NW, 4
+// to 16 waves by the context.  Workgroup b serves head b / n_kv of KV head b %
+// n_kv's group, so that the heads sharing a KV head's rows run on as few XCDs
+// as the round-robin dispatch allows (their loads meet in one L2).  A position
+// is read by HSP / 8 lanes as in the split kernel, ATTN_ONE_U positions per
+// thread and batch, the next batch's rows in flight while this one is folded
+// in; the first batch goes out before the position is known, from rows
+// clamped below the host's bound.  The position groups of a wave are summed
+// across lanes, the waves through LDS with one barrier.
+//
+// What bounds it: one memory round trip (about 2 us behind the launch) and
+// then one CU's share of the cache bandwidth (T x 512 bytes a workgroup with
+// f16 and 128 dims), so that it loses to the split kernel and its merge as T
+// grows; the host's rule and both sides' times are at launch_attn.
+template <bool F16>
+constexpr int ATTN_ONE_U = F16 ? 4 : 2;
+
+// v summed (or maximised) over the lanes that differ in bits 4 and 5, and for
+// 64 dims in bit 3 as well: every lane gets the result.  permlane16_swap and
+// permlane32_swap of (v, v) give both rows (halves) of a pair to each of its
+// lanes; row_ror 8 is lane ^ 8 within 16.
+template <int HSP, class OP>
+IFR_DEV float attn_groups_reduce(float v, OP op) {
+    if constexpr (HSP == 64)
+        v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, true)));
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(t[0]), __uint_as_float(t[1]));
+}
+
+template <int HSP, bool F16>
+__device__ void attn_one_body(const AttnArgs &a) {
+    constexpr int TPP = HSP / 8, PPW = 64 / TPP, U = ATTN_ONE_U<F16>;
+    __shared__ __attribute__((aligned(16))) float og[ATTN_ONE_WAVES][HSP];
+    __shared__ float mg[ATTN_ONE_WAVES], lg[ATTN_ONE_WAVES];
+    asm volatile("" ::"s"(a.q), "s"(a.k_cache), "s"(a.v_cache), "s"(a.out), "s"(a.xq_out), "s"(a.pos), "s"(a.kv_dim),
+                 "s"(a.seq_cap), "s"(a.spec_rows), "s"(a.head_size), "s"(a.kv_mul), "s"(a.n_out));
+    const uint32_t pos_dev = __hip_atomic_load(a.pos, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane((uint32_t)tid >> 6), nw = blockDim.x >> 6;
+    const uint32_t hs = a.head_size, G = a.kv_mul, nkv = gridDim.x / G;
+    const uint32_t kvh = blockIdx.x % nkv, h = kvh * G + blockIdx.x / nkv;
+    const uint32_t dc = (uint32_t)lane % TPP, pg = wave * PPW + (uint32_t)lane / TPP, ppp = nw * PPW;
+    const bool dim_ok = dc * 8 < hs;
+    const uint32_t dq = min(dc, hs / 8 - 1) * 8; // a lane past the head size reads its last dims and drops them
+    const float *qp = a.q + (size_t)h * hs + dq;
+    const float4 qu = *(const float4 *)qp, qw = *(const float4 *)(qp + 4);
+    const size_t head_ld = (size_t)kvh * hs + dq;
+    KV8<F16> kr[2][U], vr[2][U];
+    auto load = [&](int b, uint32_t base, uint32_t rows) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const size_t off = (size_t)min(base + pg + ppp * u, rows - 1) * a.kv_dim + head_ld;
+            if constexpr (F16) {
+                kr[b][u].u = ld16((const uint8_t *)a.k_cache + 2 * off);
+                vr[b][u].u = ld16((const uint8_t *)a.v_cache + 2 * off);
+            } else {
+                kr[b][u].u = ld16((const uint8_t *)a.k_cache + 4 * off);
+                kr[b][u].w = ld16((const uint8_t *)a.k_cache + 4 * off + 16);
+                vr[b][u].u = ld16((const uint8_t *)a.v_cache + 4 * off);
+                vr[b][u].w = ld16((const uint8_t *)a.v_cache + 4 * off + 16);
+            }
+        }
+    };
+    load(0, 0, min(a.spec_rows, a.seq_cap));
+    __builtin_amdgcn_sched_barrier(0);
+    const float sj = dim_ok ? 1.44269504088896341f / sqrtf((float)hs) : 0.0f;
+    const float q[8] = {qu.x * sj, qu.y * sj, qu.z * sj, qu.w * sj, qw.x * sj, qw.y * sj, qw.z * sj, qw.w * sj};
+    const uint32_t T = min((uint32_t)__builtin_amdgcn_readfirstlane(pos_dev) + 1u, a.seq_cap);
+    if (T > a.spec_rows) load(0, 0, T); // (uniform) a position past the host's bound
+    float m = ATTN_M0, l = 0.0f, o[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    const uint32_t step = ppp * U;
+    auto fold = [&](int b, uint32_t base) {
+        float sc[U], mb = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const bool ok = base + pg + ppp * u < T;
+            float d = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) d = fmaf(q[e], kv8_at<F16>(kr[b][u], e), d);
+            d = group_sum<TPP>(d);
+            sc[u] = ok ? d : -INFINITY;
+            mb = fmaxf(mb, sc[u]);
+            if (!ok) kv8_zero<F16>(vr[b][u]); // a row possibly never written
+        }
+        const float mn = fmaxf(m, mb), al = softmax_exp2(m - mn);
+        l *= al;
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[e] *= al;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const float p = softmax_exp2(sc[u] - mn);
+            l += p;
+#pragma unroll
+            for (int e = 0; e < 8; e++) o[e] = fmaf(p, kv8_at<F16>(vr[b][u], e), o[e]);
+        }
+        m = mn;
+    };
+    for (uint32_t base = 0; base < T; base += 2 * step) {
+        load(1, base + step, T); // past the end: the last row, masked
+        fold(0, base);
+        load(0, base + 2 * step, T);
+        if (base + step < T) fold(1, base + step);
+    }
+    // the wave's position groups, then the waves
+    const float M = attn_groups_reduce<HSP>(m, [](float x, float y) { return fmaxf(x, y); });
+    const float al = softmax_exp2(m - M);
+    auto add = [](float x, float y) { return x + y; };
+    l = attn_groups_reduce<HSP>(l * al, add);
+#pragma unroll
+    for (int e = 0; e < 8; e++) o[e] = attn_groups_reduce<HSP>(o[e] * al, add);
+    if (lane < TPP) {
+        *(float4 *)&og[wave][8 * dc] = make_float4(o[0], o[1], o[2], o[3]);
+        *(float4 *)&og[wave][8 * dc + 4] = make_float4(o[4], o[5], o[6], o[7]);
+        if (lane == 0) {
+            mg[wave] = M;
+            lg[wave] = l;
+        }
+    }
+    __syncthreads();
+    if (tid >= HSP) return;
+    float Mt = ATTN_M0, L = 0.0f, O = 0.0f;
+    for (uint32_t w = 0; w < nw; w++) Mt = fmaxf(Mt, mg[w]);
+    for (uint32_t w = 0; w < nw; w++) {
+        const float wt = softmax_exp2(mg[w] - Mt); // 0 for a wave that saw no position
+        L = fmaf(lg[w], wt, L);
+        O = fmaf(og[w][tid], wt, O);
+    }
+    const float res = O / L;
+    const bool ok = (uint32_t)tid < hs;
+    const uint32_t oi = h * hs + (uint32_t)tid;
+    if (ok && a.out) a.out[oi] = res;
+    if (a.xq_out) quant16(ok ? res : 0.0f, ok, a.xq_out, a.n_out, oi, lane); // hs % 16 == 0: whole groups
 }
 
 } // namespace ifr

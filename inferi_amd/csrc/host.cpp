@@ -395,10 +395,17 @@ static uint32_t attn_splits_for(uint32_t T, uint32_t head_size) {
     const uint32_t q = 8192u / attn_hsp(head_size);
     return std::max(1u, std::min(ATTN_SPLITS_MAX, (uint32_t)(((uint64_t)T + q - 1) / q)));
 }
-// A KV head's query heads go to n_sub workgroups of gt heads each (gt <= 8,
-// the last workgroup holding the rest).
-static void attn_groups(uint32_t kv_mul, uint32_t &n_sub, uint32_t &gt) {
-    n_sub = (kv_mul + ATTN_GT_MAX - 1) / ATTN_GT_MAX;
+// A KV head's query heads go to n_sub workgroups of gt heads each (the last
+// one holding the rest): gt at most 4 while the positions' K and V rows are
+// under 8 MB, else at most 8.  A group's heads share one pass over the rows
+// but wait for each other's arithmetic; below that size the rows' second read
+// comes from the L2 (us for split and merge, 8 or 4 heads at most: 32 heads
+// over 4 of 64 dims, f16, 1 MB 10.4 and 7.7, 4 MB 10.4 and 8.4; 12 over 2 of
+// 128, f32, 4 MB 9.8 and 9.1, 17 MB 12.3 and 13.9; 40 over 8 of 128, f16, 4 MB
+// 8.7 and 8.3, 8.4 MB 9.5 and 10.3).
+static void attn_groups(uint32_t kv_mul, uint64_t kv_bytes, uint32_t &n_sub, uint32_t &gt) {
+    const uint32_t most = kv_bytes < 8000000 ? 4 : ATTN_GT_MAX;
+    n_sub = (kv_mul + most - 1) / most;
     gt = (kv_mul + n_sub - 1) / n_sub;
 }
 
@@ -411,14 +418,35 @@ static uint32_t attn_spec_for(uint32_t pos, uint32_t max_pos) {
     return (uint32_t)std::min<uint64_t>(max_pos, ((uint64_t)pos / ATTN_BUCKET + 1) * ATTN_BUCKET);
 }
 
-// Split pass over the KV sequence, then the merge of the partials.  `a`
-// carries head_size, kv_mul, n_splits and n_out; n_sub is set here.
+// Contexts this short (spec_rows x head size padded to 64 or 128) run in one
+// kernel, a workgroup per query head (device/attention.h attn_one_body):
+// up to 1024 positions of 64 dims, 512 of 128.  Past them one CU's pass over
+// its head's rows takes longer than the split kernel with its merge (us, one
+// kernel and split + merge: 32 heads over 8 of 128, f16, 145 positions 4.5
+// and 7.7, 512 6.6 and 7.7, 778 9.6 and 7.9; 32 over 4 of 64, f16, 145 3.9
+// and 7.7, 1024 6.5 and 7.7, 2048 9.7 and 7.9; 14 over 2 of 64, f32, 1024 8.6
+// and 9.0; 12 over 2 of 128, f32, 512 8.9 and 8.8).  Its output is quantized
+// in 16-value groups of one head, so the head size is a multiple of 16.
+constexpr uint32_t ATTN_ONE_ELEMS = 65536;
+
+// Attention of one token over the cache: the one-kernel form, or the split
+// pass over the sequence and the merge of its partials.  `a` carries
+// head_size, kv_mul, n_splits, spec_rows and n_out; n_sub is set here.
 static ifr_status launch_attn(ifr_ctx *c, int32_t kv_dtype, AttnArgs &a, uint32_t n_kv_heads) {
-    uint32_t n_sub, gt;
-    attn_groups(a.kv_mul, n_sub, gt);
-    a.n_sub = n_sub;
     char name[64];
-    snprintf(name, sizeof name, "attn_%s_h%u_g%u", kv_dtype == IFR_F16 ? "f16" : "f32", attn_hsp(a.head_size), gt);
+    const char *kv = kv_dtype == IFR_F16 ? "f16" : "f32";
+    const uint32_t hsp = attn_hsp(a.head_size);
+    if (a.head_size % 16 == 0 && (uint64_t)a.spec_rows * hsp <= ATTN_ONE_ELEMS) {
+        // as many waves as one batch of the positions takes (4 or, f32, 2 per lane)
+        const uint32_t per_wave = 64 / (hsp / 8) * (kv_dtype == IFR_F16 ? 4u : 2u);
+        const uint32_t nw = std::min(ATTN_ONE_WAVES, std::max(4u, (a.spec_rows + per_wave - 1) / per_wave));
+        snprintf(name, sizeof name, "attn_one_%s_h%u", kv, hsp);
+        return c->launch(name, dim3(n_kv_heads * a.kv_mul), dim3(nw * 64), 0, a);
+    }
+    uint32_t n_sub, gt;
+    attn_groups(a.kv_mul, (uint64_t)a.spec_rows * a.kv_dim * (kv_dtype == IFR_F16 ? 4 : 8), n_sub, gt);
+    a.n_sub = n_sub;
+    snprintf(name, sizeof name, "attn_%s_h%u_g%u", kv, hsp, gt);
     ifr_status st = c->launch(name, dim3(n_kv_heads * n_sub, a.n_splits), dim3(256), 0, a);
     if (st) return st;
     return c->launch("attn_merge", dim3((a.n_out + 15) / 16), dim3(64), 0, a);

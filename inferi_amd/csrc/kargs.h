@@ -87,6 +87,10 @@ struct GemvArgs {
     int32_t neox;        // QKV: RoPE pairs (j, j + hs/2) instead of (2j, 2j+1)
 };
 
+// Decode attention in one kernel (device/attention.h attn_one_body): waves per
+// workgroup at most.
+constexpr uint32_t ATTN_ONE_WAVES = 16;
+
 struct AttnArgs {
     const float *q;           // [n_heads * head_size]
     const void *k_cache;      // [seq_len][kv_dim]

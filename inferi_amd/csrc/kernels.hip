@@ -143,6 +143,15 @@ GEMV_ALL_MODES(f32, F32)
     ATTN_KERNEL(HSP, 1, NAME, KV16) ATTN_KERNEL(HSP, 2, NAME, KV16) ATTN_KERNEL(HSP, 3, NAME, KV16) \
     ATTN_KERNEL(HSP, 5, NAME, KV16) ATTN_KERNEL(HSP, 6, NAME, KV16) ATTN_KERNEL(HSP, 7, NAME, KV16) \
     ATTN_KERNEL(HSP, 8, NAME, KV16)
+// and in one kernel, one query head per workgroup (short contexts)
+#define ATTN_ONE_KERNEL(HSP, NAME, KV16)                                                            \
+    extern "C" __global__ void __launch_bounds__(ATTN_ONE_WAVES * 64) attn_one_##NAME##_h##HSP(AttnArgs a) { \
+        attn_one_body<HSP, KV16>(a);                                                    \
+    }
+ATTN_ONE_KERNEL(64, f16, true)
+ATTN_ONE_KERNEL(128, f16, true)
+ATTN_ONE_KERNEL(64, f32, false)
+ATTN_ONE_KERNEL(128, f32, false)
 ATTN_KERNELS(64, f16, true)
 ATTN_KERNEL(64, 4, f16, true)
 ATTN_KERNELS(64, f32, false)

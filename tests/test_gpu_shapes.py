@@ -296,3 +296,19 @@ def test_decode_position_buckets(ctx, oracle_lib):
                 s.close()
     finally:
         w.close()
+
+
+@pytest.mark.parametrize("kv_f16", [True, False], ids=["f16", "f32"])
+@pytest.mark.parametrize("nh,nkv,hs", [(7, 1, 16), (6, 2, 48), (14, 2, 64), (10, 2, 80), (8, 8, 112), (40, 8, 128)])
+def test_attention_one_kernel_edges(ctx, oracle_lib, kv_f16, nh, nkv, hs):
+    """The one-kernel form at the edges of its waves and batches, on both
+    sides of the context where the split kernel takes over (1024 positions of
+    up to 64 dims, 512 of up to 128), with head sizes short of the padding,
+    and the split kernel's sub-groups of at most four heads past it.  The
+    outputs are averages of at most 1025 N(0, 1) values in f32: 1e-5 leaves
+    twenty times the largest difference two summation orders show."""
+    rng = np.random.default_rng(nh * 100 + hs)
+    top = 1024 if hs <= 64 else 512
+    for T in (2, 31, 32, 33, 129, 256, 257, top - 1, top, top + 1):
+        got, ref = _attn_case(ctx, nh, nkv, hs, top + 1, T - 1, kv_f16, rng)
+        assert np.abs(got - ref).max() <= 1e-5, f"{T} positions"
