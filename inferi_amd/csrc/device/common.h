@@ -12,6 +12,10 @@
 namespace ifr {
 
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+// at the alignments GGUF fields have: global loads need none on gfx950
+// (unaligned access mode), and the compiler emits one load for each
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32_a2 __attribute__((aligned(2)));
 // matrix-core operand and accumulator vectors (v_mfma_f32_32x32x16_f16)
 typedef _Float16 half8v __attribute__((ext_vector_type(8)));
 typedef float float16v __attribute__((ext_vector_type(16)));

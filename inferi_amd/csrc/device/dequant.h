@@ -14,18 +14,23 @@ namespace ifr {
 
 IFR_DEV uint32_t rd8(const uint8_t *p) { return *p; }
 
+// Header of a Q4_K or Q5_K block (d@0 dmin@2 scales[12]@4): d * sc and dmin *
+// m of sub-block j.
+IFR_DEV void k4_header(const uint8_t *blk, uint32_t j, float &d1, float &m1) {
+#pragma clang fp contract(off)
+    const u32x4_a2 h = *(const u32x4_a2 *)blk;
+    uint32_t sc, m;
+    scale_min_k4(j, h.y, h.z, h.w, sc, m);
+    d1 = f16_to_f32(h.x & 0xFFFFu) * (float)sc;
+    m1 = f16_to_f32(h.x >> 16) * (float)m;
+}
+
 // Q4_K: d@0 dmin@2 scales[12]@4 qs[128]@16; element e = 64g + 32hi + l.
 IFR_DEV float deq_q4k(const uint8_t *blk, uint32_t e) {
 #pragma clang fp contract(off)
     uint32_t g = e >> 6, hi = (e >> 5) & 1u, l = e & 31u;
-    float d = f16_to_f32(ld_u16(blk)), dmin = f16_to_f32(ld_u16(blk + 2));
-    const uint8_t *s = blk + 4;
-    uint32_t w0 = rd8(s) | rd8(s + 1) << 8 | rd8(s + 2) << 16 | rd8(s + 3) << 24;
-    uint32_t w1 = rd8(s + 4) | rd8(s + 5) << 8 | rd8(s + 6) << 16 | rd8(s + 7) << 24;
-    uint32_t w2 = rd8(s + 8) | rd8(s + 9) << 8 | rd8(s + 10) << 16 | rd8(s + 11) << 24;
-    uint32_t sc, m;
-    scale_min_k4(2 * g + hi, w0, w1, w2, sc, m);
-    float d1 = d * (float)sc, m1 = dmin * (float)m;
+    float d1, m1;
+    k4_header(blk, 2 * g + hi, d1, m1);
     uint32_t q = rd8(blk + 16 + 32 * g + l);
     q = hi ? (q >> 4) : (q & 15u);
     return d1 * (float)q - m1;
@@ -35,14 +40,8 @@ IFR_DEV float deq_q4k(const uint8_t *blk, uint32_t e) {
 IFR_DEV float deq_q5k(const uint8_t *blk, uint32_t e) {
 #pragma clang fp contract(off)
     uint32_t g = e >> 6, hi = (e >> 5) & 1u, l = e & 31u;
-    float d = f16_to_f32(ld_u16(blk)), dmin = f16_to_f32(ld_u16(blk + 2));
-    const uint8_t *s = blk + 4;
-    uint32_t w0 = rd8(s) | rd8(s + 1) << 8 | rd8(s + 2) << 16 | rd8(s + 3) << 24;
-    uint32_t w1 = rd8(s + 4) | rd8(s + 5) << 8 | rd8(s + 6) << 16 | rd8(s + 7) << 24;
-    uint32_t w2 = rd8(s + 8) | rd8(s + 9) << 8 | rd8(s + 10) << 16 | rd8(s + 11) << 24;
-    uint32_t sc, m;
-    scale_min_k4(2 * g + hi, w0, w1, w2, sc, m);
-    float d1 = d * (float)sc, m1 = dmin * (float)m;
+    float d1, m1;
+    k4_header(blk, 2 * g + hi, d1, m1);
     uint32_t q = rd8(blk + 48 + 32 * g + l);
     q = hi ? (q >> 4) : (q & 15u);
     uint32_t h = (rd8(blk + 16 + l) >> (2 * g + hi)) & 1u;
@@ -159,6 +158,93 @@ IFR_DEV float deq_elem(int fmt, const uint8_t *base, uint64_t idx) {
     case Q5_K: return deq_q5k(blk, e);
     case Q8_K: return deq_q8_k(blk, e);
     default: return deq_q6k(blk, e);
+    }
+}
+
+// Elements idx .. idx + 3 (idx a multiple of 4; the formats' runs of equal
+// scales and their code bytes come in fours at least) of a tensor stored as
+// consecutive blocks: the same values as deq_elem, the codes of four elements
+// in one load and the header in one.
+template <int FMT>
+IFR_DEV void deq4(const uint8_t *base, uint64_t idx, float (&y)[4]) {
+#pragma clang fp contract(off)
+    auto code = [](uint32_t w, int k) { return (w >> (8 * k)) & 0xFFu; };
+    if constexpr (FMT == F32) {
+        const u32x4_a4 v = *(const u32x4_a4 *)(base + 4 * idx);
+#pragma unroll
+        for (int k = 0; k < 4; k++) y[k] = __uint_as_float(v[k]);
+    } else if constexpr (FMT == F16) {
+        const uint32_t a = *(const u32_a2 *)(base + 2 * idx), b = *(const u32_a2 *)(base + 2 * idx + 4);
+        y[0] = f16_to_f32(a & 0xFFFFu);
+        y[1] = f16_to_f32(a >> 16);
+        y[2] = f16_to_f32(b & 0xFFFFu);
+        y[3] = f16_to_f32(b >> 16);
+    } else if constexpr (FMT == Q4_K || FMT == Q5_K) {
+        const uint32_t e = (uint32_t)idx & 255u, g = e >> 6, hi = (e >> 5) & 1u, l = e & 31u;
+        const uint8_t *blk = base + (idx >> 8) * (FMT == Q4_K ? 144u : 176u);
+        uint32_t w = *(const u32_a2 *)(blk + (FMT == Q4_K ? 16 : 48) + 32 * g + l);
+        w = (hi ? w >> 4 : w) & 0x0F0F0F0Fu;
+        if constexpr (FMT == Q5_K) w |= ((*(const u32_a2 *)(blk + 16 + l) >> (2 * g + hi)) & 0x01010101u) << 4;
+        float d1, m1;
+        k4_header(blk, 2 * g + hi, d1, m1);
+#pragma unroll
+        for (int k = 0; k < 4; k++) y[k] = d1 * (float)code(w, k) - m1;
+    } else if constexpr (FMT == Q6_K) {
+        const uint32_t e = (uint32_t)idx & 255u, i = e >> 7, k2 = (e >> 5) & 3u, l = e & 31u;
+        const uint8_t *blk = base + (idx >> 8) * 210u;
+        uint32_t w = *(const u32_a2 *)(blk + 64 * i + l + 32 * (k2 & 1u));
+        w = (k2 < 2 ? w : w >> 4) & 0x0F0F0F0Fu;
+        w |= ((*(const u32_a2 *)(blk + 128 + 32 * i + l) >> (2 * k2)) & 0x03030303u) << 4;
+        const float s = f16_to_f32(ld_u16(blk + 208)) * (float)(int)(int8_t)rd8(blk + 192 + 8 * i + (l >> 4) + 2 * k2);
+#pragma unroll
+        for (int k = 0; k < 4; k++) y[k] = s * (float)((int)code(w, k) - 32);
+    } else if constexpr (FMT == Q8_K) {
+        const uint8_t *blk = base + (idx >> 8) * 292u;
+        const uint32_t w = *(const u32_a2 *)(blk + 4 + ((uint32_t)idx & 255u));
+        const float d = *(const float *)blk;
+#pragma unroll
+        for (int k = 0; k < 4; k++) y[k] = d * (float)(int)(int8_t)code(w, k);
+    } else {
+        constexpr uint32_t QS = FMT == Q4_0 || FMT == Q8_0 ? 2 : FMT == Q4_1 ? 4 : FMT == Q5_0 ? 6 : 8;
+        constexpr uint32_t BB = FMT == Q8_0 ? 34 : QS + 16;
+        const uint32_t e = (uint32_t)idx & 31u;
+        const uint8_t *blk = base + (idx >> 5) * BB;
+        const float d = f16_to_f32(ld_u16(blk));
+        if constexpr (FMT == Q8_0) {
+            const uint32_t w = *(const u32_a2 *)(blk + QS + e);
+#pragma unroll
+            for (int k = 0; k < 4; k++) y[k] = (float)(int)(int8_t)code(w, k) * d;
+        } else {
+            uint32_t w = *(const u32_a2 *)(blk + QS + (e & 15u));
+            w = (e < 16 ? w : w >> 4) & 0x0F0F0F0Fu;
+            if constexpr (FMT == Q5_0 || FMT == Q5_1) w |= spread4_b4((*(const u32_a2 *)(blk + QS - 4) >> e) & 15u);
+            const float m = FMT == Q4_1 || FMT == Q5_1 ? f16_to_f32(ld_u16(blk + 2)) : 0.0f;
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                y[k] = FMT == Q4_1 || FMT == Q5_1 ? (float)code(w, k) * d + m
+                                                  : (float)((int)code(w, k) - (FMT == Q4_0 ? 8 : 16)) * d;
+        }
+    }
+}
+// f(integral constant of a type) for the type `fmt`.
+template <int FMT>
+struct FmtC {
+    static constexpr int value = FMT;
+};
+template <class F>
+IFR_DEV void with_fmt(int fmt, F f) {
+    switch (fmt) {
+    case F32: f(FmtC<F32>{}); break;
+    case F16: f(FmtC<F16>{}); break;
+    case Q4_0: f(FmtC<Q4_0>{}); break;
+    case Q4_1: f(FmtC<Q4_1>{}); break;
+    case Q5_0: f(FmtC<Q5_0>{}); break;
+    case Q5_1: f(FmtC<Q5_1>{}); break;
+    case Q8_0: f(FmtC<Q8_0>{}); break;
+    case Q4_K: f(FmtC<Q4_K>{}); break;
+    case Q5_K: f(FmtC<Q5_K>{}); break;
+    case Q8_K: f(FmtC<Q8_K>{}); break;
+    default: f(FmtC<Q6_K>{}); break;
     }
 }
 

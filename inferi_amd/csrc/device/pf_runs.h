@@ -67,8 +67,6 @@ typedef _Float16 f16x2v __attribute__((ext_vector_type(2)));
 //    rounding to f16 is the only one, and v_pk_mul_f16 of the exact f16
 //    integer c - z rounds the same product once (pg_pk4).
 // Two-byte aligned fields are read with the hardware's unaligned loads.
-typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
-typedef uint32_t u32_a2 __attribute__((aligned(2)));
 
 // Four codes, the bytes of c: y = s c + o, s given times 2^24, as two f16 pairs.
 IFR_DEV void pg_mix4(uint32_t c, float s24, float o, uint32_t &u0, uint32_t &u1) {

@@ -18,14 +18,19 @@ namespace ifr {
 
 // ------------------------------------------------------------ pointwise --
 
-// X[m] = dequant(table)[tok[p0 + m]]
+// X[m] = dequant(table)[tok[p0 + m]], four elements per thread and turn
 IFR_DEV void pf_embed_body(const PfArgs &a) {
-    float *xo = (float *)a.x;
     const uint32_t m = blockIdx.x;
-    const uint32_t tok = a.tokens[a.p0 + m];
-    const uint8_t *row = a.table + (size_t)tok * a.row_bytes;
-    for (uint32_t i = threadIdx.x; i < a.hidden; i += blockDim.x)
-        xo[(size_t)m * a.hidden + i] = deq_elem(a.fmt, row, i);
+    float *xo = (float *)a.x + (size_t)m * a.hidden;
+    const uint8_t *row = a.table + (size_t)a.tokens[a.p0 + m] * a.row_bytes;
+    with_fmt(a.fmt, [&](auto f) {
+        constexpr int FMT = decltype(f)::value;
+        for (uint32_t i = 4 * threadIdx.x; i < a.hidden; i += 4 * blockDim.x) {
+            float y[4];
+            deq4<FMT>(row, i, y);
+            *(float4 *)(xo + i) = make_float4(y[0], y[1], y[2], y[3]);
+        }
+    });
 }
 
 // xh[m] = f16((x[m] * (1/sqrt(mean(x[m]^2) + eps))) * gamma), rms_norm.rs:81-121

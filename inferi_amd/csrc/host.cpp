@@ -1126,7 +1126,7 @@ IFR_API ifr_status ifr_dequant(ifr_ctx *c, float *out, const void *blocks, int32
     // f32 fields (F32, Q8_K's d) need 4-byte alignment, f16 fields 2
     if ((uintptr_t)blocks % ((dtype == IFR_F32 || dtype == IFR_Q8_K) ? 4 : 2)) return c->fail(IFR_EINVAL, "dequant: misaligned blocks");
     DequantArgs a{out, (const uint8_t *)blocks, n, dtype, 0};
-    const uint64_t g = std::min<uint64_t>((n + 255) / 256, 65536);
+    const uint64_t g = std::min<uint64_t>((n + 4095) / 4096, 65536); // 16 elements per thread
     return c->launch("dequant_k", dim3((uint32_t)g), dim3(256), 0, a);
 }
 
