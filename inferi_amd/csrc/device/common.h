@@ -113,8 +113,9 @@ IFR_DEV uint4 ld16(const uint8_t *p) {
 // 16 bytes at a 2-byte aligned address, read with naturally aligned loads
 // that never leave [p, p+16): one dword-aligned 16-byte load from p & ~3 and
 // one 2-byte load for the tail when p is not dword aligned, then a funnel
-// shift.  (Q6_K blocks are 210 bytes and Q8_0 blocks 34, so their fields sit
-// at 2-byte alignment.)
+// shift.  For the formats of 18 to 34 bytes a block, whose lanes read
+// neighbouring blocks: there one unaligned load (ld16_u2) is slower (Q8_0
+// GEMV, 14336 x 4096: 18.4 us, 22.9 unaligned; Q5_0 20.3 and 24.9).
 IFR_DEV uint4 ld16_a2(const uint8_t *p) {
     uintptr_t a = (uintptr_t)p;
     uint32_t sb = (uint32_t)(a & 3u); // 0 or 2
@@ -127,6 +128,18 @@ IFR_DEV uint4 ld16_a2(const uint8_t *p) {
     r.z = __builtin_amdgcn_alignbyte(w.w, w.z, sb);
     r.w = __builtin_amdgcn_alignbyte(tail, w.w, sb);
     return r;
+}
+// The same in one unaligned load: for Q6_K, whose lanes read runs of 64 to 128
+// bytes of a 210-byte block (GEMV 128256 x 4096: 124 us with ld16_a2, 104).
+IFR_DEV uint4 ld16_u2(const uint8_t *p) {
+    const u32x4_a2 v = *(const u32x4_a2 *)p;
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+IFR_DEV uint2 ld8_u2(const uint8_t *p) {
+    typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+    const u32x2_a2 v = *(const u32x2_a2 *)p;
+    return make_uint2(v.x, v.y);
 }
 
 // 16 bytes at a 4-byte aligned address.

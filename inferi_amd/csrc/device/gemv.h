@@ -247,8 +247,8 @@ struct Chunk<Q6_K, R> {
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const uint8_t *b = rowp[r] + (size_t)kb * 210;
-            qlv[r] = ld16_a2(b + 64 * i + 16 * cp);
-            qhv[r] = ld16_a2(b + 128 + 32 * i + 16 * s);
+            qlv[r] = ld16_u2(b + 64 * i + 16 * cp);
+            qhv[r] = ld16_u2(b + 128 + 32 * i + 16 * s);
             scl[r] = b[192 + 8 * i + s + 2 * u];
             sch[r] = b[192 + 8 * i + s + 2 * u + 4];
             dsc[r] = ld_u16(b + 208);
@@ -662,18 +662,18 @@ struct ChunkI<Q6_K, R> {
     static constexpr int LPB = 4;
     static constexpr bool DIRECT = false;
     uint4 l0[R], l1[R], h0[R], h1[R];
-    uint32_t sc_lo[R], sc_hi[R], dd[R];
+    uint2 sc[R]; // scales of half i
+    uint32_t dd[R];
     IFR_DEV void load(const uint8_t *const *rowp, uint32_t kb, uint32_t c) {
         const uint32_t i = c >> 1, u = c & 1u;
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const uint8_t *b = rowp[r] + (size_t)kb * 210;
-            l0[r] = ld16_a2(b + 64 * i + 32 * u);
-            l1[r] = ld16_a2(b + 64 * i + 32 * u + 16);
-            h0[r] = ld16_a2(b + 128 + 32 * i);
-            h1[r] = ld16_a2(b + 144 + 32 * i);
-            sc_lo[r] = ld_u16(b + 192 + 8 * i + 2 * u);
-            sc_hi[r] = ld_u16(b + 196 + 8 * i + 2 * u);
+            l0[r] = ld16_u2(b + 64 * i + 32 * u);
+            l1[r] = ld16_u2(b + 64 * i + 32 * u + 16);
+            h0[r] = ld16_u2(b + 128 + 32 * i);
+            h1[r] = ld16_u2(b + 144 + 32 * i);
+            sc[r] = ld8_u2(b + 192 + 8 * i);
             dd[r] = ld_u16(b + 208);
         }
     }
@@ -698,7 +698,7 @@ struct ChunkI<Q6_K, R> {
                                     (n.z & M) | (((h.z >> sh) << 4) & B), (n.w & M) | (((h.w >> sh) << 4) & B));
         return gdot_u(cd, xg);
     }
-    IFR_DEV void combine(uint32_t, const int (&iv)[4][R], const XS4 &f, bool valid, float *acc) const {
+    IFR_DEV void combine(uint32_t c, const int (&iv)[4][R], const XS4 &f, bool valid, float *acc) const {
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const float t0 = fmaf((float)iv[0][r], f.s.x, -32.0f * f.S.x);
@@ -706,8 +706,9 @@ struct ChunkI<Q6_K, R> {
             const float t2 = fmaf((float)iv[2][r], f.s.z, -32.0f * f.S.z);
             const float t3 = fmaf((float)iv[3][r], f.s.w, -32.0f * f.S.w);
             const float d = f16_to_f32(dd[r]);
-            const float c0 = (float)(int)(int8_t)(sc_lo[r] & 0xFFu), c1 = (float)(int)(int8_t)(sc_lo[r] >> 8);
-            const float c2 = (float)(int)(int8_t)(sc_hi[r] & 0xFFu), c3 = (float)(int)(int8_t)(sc_hi[r] >> 8);
+            const uint32_t sc_lo = sc[r].x >> (16 * (c & 1u)), sc_hi = sc[r].y >> (16 * (c & 1u));
+            const float c0 = (float)(int)(int8_t)(sc_lo & 0xFFu), c1 = (float)(int)(int8_t)(sc_lo >> 8);
+            const float c2 = (float)(int)(int8_t)(sc_hi & 0xFFu), c3 = (float)(int)(int8_t)(sc_hi >> 8);
             const float v = d * (c0 * t0 + c1 * t1 + c2 * t2 + c3 * t3);
             acc[r] += valid ? v : 0.0f;
         }
