@@ -592,10 +592,15 @@ static ifr_status enqueue_layer(ifr_ctx *c, ifr_llama2_state *s, const ifr_llama
     const bool fuse_qkv = fused != 0;
     const bool fuse_ffn = fused && Lw.ffn_gate.dtype == Lw.ffn_up.dtype;
     // gate/up as one item per wave with h in f32, quantized by the down
-    // GEMV itself (Q4_K, rows of one K step; option gemv_grp bit 5)
+    // GEMV itself (gate rows of one K step; option gemv_grp bit 5).  Against
+    // the looping form with h quantized behind a barrier, us per step of six
+    // layers: Q8_0, hidden 896 178 -> 172; Q5_K, 2048 233 -> 216; Q6_K, 4096
+    // 527 -> 500.
+    const std::string gu_fmt = std::string("gemv_") + (fuse_ffn ? gemv_fmt_name(Lw.ffn_gate.dtype) : "") + "_gateup_one";
+    const std::string down_xf = std::string("gemv_") + gemv_fmt_name(Lw.ffn_down.dtype) + "_resid_xf";
     const bool h32 = fuse_ffn && (c->gemv_grp & 32) && !c->gemv_exact && !c->gemv_waves && !c->gemv_max_grid &&
-                     Lw.ffn_gate.dtype == IFR_Q4_K && Lw.ffn_down.dtype == IFR_Q4_K && hidden <= 4096 &&
-                     hidden % 256 == 0 && c->fn("gemv_q4_k_gateup_one") && c->fn("gemv_q4_k_resid_xf");
+                     hidden % (uint32_t)gemv_qk(Lw.ffn_gate.dtype) == 0 &&
+                     hidden / (uint32_t)gemv_qk(Lw.ffn_gate.dtype) <= int_blocks_per_step(Lw.ffn_gate.dtype);
     const float *next_norm = (const float *)(l + 1 < L ? w->layers[l + 1].attn_norm.data : w->output_norm.data);
     GemvPlan p;
 
@@ -757,10 +762,11 @@ static ifr_status enqueue_layer(ifr_ctx *c, ifr_llama2_state *s, const ifr_llama
                 a.xq_out = nullptr;
                 a.ks = 1;
                 a.nwaves = GEMV_ONE_WAVES;
-                const bool four = (c->gemv_grp & 128) && c->fn("gemv_q4_k_gateup_one4");
+                // Q4_K has the two-row form as well (bit 7 off)
+                const bool four = (c->gemv_grp & 128) || Lw.ffn_gate.dtype != IFR_Q4_K;
                 const uint32_t rows_per = GEMV_ONE_WAVES * (four ? 4 : 2), g = (a.total_rows + rows_per - 1) / rows_per;
-                if ((st = c->launch(four ? "gemv_q4_k_gateup_one4" : "gemv_q4_k_gateup_one", dim3(g),
-                                    dim3(GEMV_ONE_WAVES * 64), (uint32_t)xq_bytes(a.cols), a)))
+                if ((st = c->launch(gu_fmt + (four ? "4" : ""), dim3(g), dim3(GEMV_ONE_WAVES * 64),
+                                    (uint32_t)xq_bytes(a.cols), a)))
                     return st;
             } else if ((st = launch_gemv(c, p, "gateup", a))) {
                 return st;
@@ -805,7 +811,7 @@ static ifr_status enqueue_layer(ifr_ctx *c, ifr_llama2_state *s, const ifr_llama
                 const IntGeom g = int_geom(c, p.bpi, "resid", a, 0);
                 a.ks = g.ks;
                 a.nwaves = g.waves;
-                if ((st = c->launch("gemv_q4_k_resid_xf", dim3(g.grid), dim3(g.waves * 64), (uint32_t)xq_bytes(a.cols), a)))
+                if ((st = c->launch(down_xf, dim3(g.grid), dim3(g.waves * 64), (uint32_t)xq_bytes(a.cols), a)))
                     return st;
             } else if ((st = launch_gemv(c, p, "resid", a))) {
                 return st;

@@ -101,6 +101,17 @@ GEMV_GRP_KERNEL(gemv_q4_k_gateup, Q4_K, GEMV_GATEUP, 2, 16, 1)
         gemv_int_body<FMT, GEMV_PLAIN, GEMV_INT_PIPE, GEMV_INT_NI, true>(a);                         \
     }
 
+// gate/up with h in f32, four rows per wave, and the down GEMV that quantizes
+// its f32 input itself (Q4_K's are at the top)
+#define GEMV_H32_KERNELS(FMTNAME, FMT)                                                                     \
+    extern "C" __global__ void __launch_bounds__(GEMV_ONE_WAVES * 64) gemv_##FMTNAME##_gateup_one4(GemvArgs a) { \
+        gemv_one_body<FMT, GEMV_GATEUP, 4>(a);                                                             \
+    }                                                                                                      \
+    extern "C" __global__ void __launch_bounds__(GEMV_INT_MAX_WAVES * 64)                                  \
+        __attribute__((amdgpu_waves_per_eu(GEMV_INT_WPE, 8))) gemv_##FMTNAME##_resid_xf(GemvArgs a) {      \
+        gemv_int_body<FMT, GEMV_RESID, GEMV_INT_PIPE, GEMV_INT_NI, true>(a);                               \
+    }
+
 #define GEMV_ALL_MODES(FMTNAME, FMT)                  \
     GEMV_ONE_KERNEL(gemv_##FMTNAME##_plain, FMT, GEMV_PLAIN) \
     GEMV_ONE_XF_KERNEL(gemv_##FMTNAME##_plain, FMT)          \
@@ -114,24 +125,34 @@ GEMV_GRP_KERNEL(gemv_q4_k_gateup, Q4_K, GEMV_GATEUP, 2, 16, 1)
 
 GEMV_ALL_MODES(q4_k, Q4_K)
 GEMV_ONE_KERNEL(gemv_q5_k_qkv, Q5_K, GEMV_QKV)
+GEMV_H32_KERNELS(q5_k, Q5_K)
 GEMV_ALL_MODES(q5_k, Q5_K)
 GEMV_ONE_KERNEL(gemv_q6_k_qkv, Q6_K, GEMV_QKV)
+GEMV_H32_KERNELS(q6_k, Q6_K)
 GEMV_ALL_MODES(q6_k, Q6_K)
 GEMV_ONE_KERNEL(gemv_q8_0_qkv, Q8_0, GEMV_QKV)
+GEMV_H32_KERNELS(q8_0, Q8_0)
 GEMV_ALL_MODES(q8_0, Q8_0)
 GEMV_ONE_KERNEL(gemv_q4_0_qkv, Q4_0, GEMV_QKV)
+GEMV_H32_KERNELS(q4_0, Q4_0)
 GEMV_ALL_MODES(q4_0, Q4_0)
 GEMV_ONE_KERNEL(gemv_q4_1_qkv, Q4_1, GEMV_QKV)
+GEMV_H32_KERNELS(q4_1, Q4_1)
 GEMV_ALL_MODES(q4_1, Q4_1)
 GEMV_ONE_KERNEL(gemv_q5_0_qkv, Q5_0, GEMV_QKV)
+GEMV_H32_KERNELS(q5_0, Q5_0)
 GEMV_ALL_MODES(q5_0, Q5_0)
 GEMV_ONE_KERNEL(gemv_q5_1_qkv, Q5_1, GEMV_QKV)
+GEMV_H32_KERNELS(q5_1, Q5_1)
 GEMV_ALL_MODES(q5_1, Q5_1)
 GEMV_ONE_KERNEL(gemv_q8_k_qkv, Q8_K, GEMV_QKV)
+GEMV_H32_KERNELS(q8_k, Q8_K)
 GEMV_ALL_MODES(q8_k, Q8_K)
 GEMV_ONE_KERNEL(gemv_f16_qkv, F16, GEMV_QKV)
+GEMV_H32_KERNELS(f16, F16)
 GEMV_ALL_MODES(f16, F16)
 GEMV_ONE_KERNEL(gemv_f32_qkv, F32, GEMV_QKV)
+GEMV_H32_KERNELS(f32, F32)
 GEMV_ALL_MODES(f32, F32)
 
 // decode attention: head sizes padded to 64 or 128, 1..8 query heads per workgroup

@@ -89,3 +89,40 @@ def test_matmul_quant_four_row_form(ctx, dtype_name, rows, cols):
     finally:
         for b in (dw, dx, y):
             b.free()
+
+
+@pytest.mark.parametrize("gate,down,hidden,ffn", [
+    ("Q8_0", "Q8_0", 1024, 544), ("Q8_0", "Q4_0", 1056, 544), ("Q4_0", "Q5_1", 896, 1056), ("Q4_1", "Q5_0", 32, 96),
+    ("Q5_0", "F16", 64, 288), ("Q5_1", "F32", 1024, 32), ("F16", "Q8_0", 992, 320), ("F32", "Q4_1", 288, 1024),
+    ("Q5_K", "Q6_K", 4096, 256), ("Q6_K", "Q5_K", 4096, 768), ("Q6_K", "Q8_K", 4352, 512), ("Q8_K", "Q4_K", 512, 1280),
+    ("Q4_K", "Q6_K", 2048, 512)])
+def test_ffn_f32_hidden_every_type(ctx, gate, down, hidden, ffn):
+    """The gate/up form that leaves h in f32 with the down GEMV that quantizes
+    it, for each type and for gate and down of different types, at one K step
+    (32-element types up to 1024, K-quants up to 4096), just past it (the
+    looping form) and with ragged FFN widths: the fused step's logits against
+    the one-op-per-kernel step's on the same weights.  Both take x as 22-bit
+    codes; they differ in the order of f32 sums only, 1e-5 of the largest
+    logit (the bar is ten times that)."""
+    import inferi_amd as I
+
+    heads = next(h for h in range(1, 200) if hidden % (8 * h) == 0 and hidden // h <= 128)
+    cfg = I.Llama2Config(n_layers=2, hidden=hidden, ffn=ffn, n_heads=heads, n_kv_heads=heads, vocab=256, max_pos=16,
+                         rope_theta=10000.0, rms_eps=1e-5, kv_dtype=I.F32)
+    mats = {"ffn_gate": getattr(I, gate), "ffn_up": getattr(I, gate), "ffn_down": getattr(I, down)}
+    # the other matrices in a type that any width takes
+    w = I.Llama2Weights.synthetic(ctx, cfg, seed=hidden + ffn, mat_dtype=I.Q8_0, head_dtype=I.Q8_0, embd_dtype=I.Q8_0,
+                                  std=0.05, overrides=mats)
+    logits = {}
+    try:
+        for fused in (True, False):
+            s = I.Llama2State(ctx, cfg)
+            s.reset([3, 250, 17, 99], 0)
+            for _ in range(4):
+                I.Llama2.launch(ctx, s, w, fused)
+            logits[fused] = s.read("logits").astype(np.float64)
+            s.close()
+    finally:
+        w.close()
+    err = np.abs(logits[True] - logits[False]).max() / np.abs(logits[False]).max()
+    assert err <= 1e-4, f"{err:.2e}"
