@@ -191,6 +191,13 @@ __device__ void quant_act_body(const QActArgs &a) {
     if (tid == 0 && a.ss_out) a.ss_out[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
+__device__ void set_pos_body(const SetPosArgs &a) {
+    const uint32_t t = threadIdx.x;
+    if (t == 0) *a.ctl = a.ctl_v;
+    if (t < 4) ((uint32_t *)a.rope)[t] = a.rope_v[t];
+    if (t < 6) ((uint32_t *)a.attn)[t] = a.attn_v[t];
+}
+
 // cache[pos] <- k, v (rounded to binary16 when kv_f16).
 __device__ void kv_store_body(const KvStoreArgs &a) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;

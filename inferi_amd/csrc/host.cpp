@@ -112,6 +112,13 @@ struct ifr_ctx {
     hipStream_t stream = nullptr;
     hipModule_t module = nullptr;
     std::map<std::string, hipFunction_t> fns;
+    // kernels of ifr_matmul_quant's f32 input by type id: rows of one K step
+    // and longer ones (looked up at a type's first call)
+    struct PlainXf {
+        bool known = false;
+        hipFunction_t one = nullptr, loop = nullptr;
+    } plain_xf[16];
+    StepCtl *ctl_host = nullptr; // pinned: a state's control block read back
     std::string err;
     char dev_name[256] = {0};
     int n_cu = 0;
@@ -171,7 +178,10 @@ struct ifr_ctx {
         auto it = fns.find(name);
         if (it != fns.end()) return it->second;
         hipFunction_t f = nullptr;
-        if (hipModuleGetFunction(&f, module, name.c_str()) != hipSuccess) f = nullptr;
+        if (hipModuleGetFunction(&f, module, name.c_str()) != hipSuccess) {
+            f = nullptr;
+            hipGetLastError(); // a form that a type does not have: not left for the program's next HIP call
+        }
         fns[name] = f;
         return f;
     }
@@ -179,12 +189,15 @@ struct ifr_ctx {
     ifr_status launch(const std::string &name, dim3 grid, dim3 block, uint32_t shmem, const A &args) {
         hipFunction_t f = fn(name);
         if (!f) return fail(IFR_EUNSUPPORTED, "kernel %s not in the code object", name.c_str());
+        return launch_fn(f, name.c_str(), grid, block, shmem, args);
+    }
+    template <class A>
+    ifr_status launch_fn(hipFunction_t f, const char *name, dim3 grid, dim3 block, uint32_t shmem, const A &args) {
         // every kernel takes one struct argument: kernelParams[0] points at it
-        A copy = args;
-        void *params[] = {&copy};
+        void *params[] = {const_cast<A *>(&args)};
         return hip(hipModuleLaunchKernel(f, grid.x, grid.y, grid.z, block.x, block.y, block.z, shmem, stream, params,
                                          nullptr),
-                   name.c_str());
+                   name);
     }
     ifr_status ensure_xq_scratch(size_t bytes) {
         if (bytes <= xq_scratch_bytes) return IFR_OK;
@@ -276,10 +289,8 @@ static IntGeom int_geom(const ifr_ctx *c, uint32_t bpi, const char *mode, const 
     return g;
 }
 
-// xf (plain mode only): a.x is f32 and the kernel quantizes it into its LDS
-// itself (the `_xf` forms), instead of reading a.xq.
 static ifr_status launch_gemv(ifr_ctx *c, const GemvPlan &p, const char *mode, GemvArgs &a, uint32_t cap = 0,
-                              uint32_t *grid_out = nullptr, bool xf = false) {
+                              uint32_t *grid_out = nullptr) {
     const bool exact = c->gemv_exact != 0;
     std::string name = std::string("gemv_") + p.fmt + "_" + mode + (exact ? "_f32" : "");
     if (exact) {
@@ -292,7 +303,7 @@ static ifr_status launch_gemv(ifr_ctx *c, const GemvPlan &p, const char *mode, G
         if (grid_out) *grid_out = g;
         return c->launch(name, dim3(g), dim3((uint32_t)ge.W * 64u), a.cols * 4, a);
     }
-    if ((!xf && !a.xq) || (a.total_rows && a.cols % 16))
+    if (!a.xq || (a.total_rows && a.cols % 16))
         return c->fail(IFR_EINVAL, "gemv: integer path needs a quantized input");
     // plain and qkv rows of one 64-lane step: the one-item kernel, every
     // workgroup launched at once
@@ -301,12 +312,12 @@ static ifr_status launch_gemv(ifr_ctx *c, const GemvPlan &p, const char *mode, G
         // four rows per wave where the code object has that form (bit 8;
         // slower for the QKV launch's 6144 rows, whose 384 workgroups of
         // four-row waves do not fill the chip)
-        const bool four = !xf && (c->gemv_grp & 256) && c->fn(name + "_one4");
+        const bool four = (c->gemv_grp & 256) && c->fn(name + "_one4");
         const uint32_t rows_per = GEMV_ONE_WAVES * (four ? 4 : 2), g = (a.total_rows + rows_per - 1) / rows_per;
         a.ks = 1;
         a.nwaves = GEMV_ONE_WAVES;
         if (grid_out) *grid_out = g;
-        return c->launch(name + (four ? "_one4" : xf ? "_one_xf" : "_one"), dim3(g), dim3(GEMV_ONE_WAVES * 64),
+        return c->launch(name + (four ? "_one4" : "_one"), dim3(g), dim3(GEMV_ONE_WAVES * 64),
                          (uint32_t)xq_bytes(a.cols), a);
     }
     // resid and gateup: one output group per workgroup, one item per wave,
@@ -342,7 +353,7 @@ static ifr_status launch_gemv(ifr_ctx *c, const GemvPlan &p, const char *mode, G
         if (grid_out) *grid_out = gg;
         return c->launch(name + "_w2", dim3(gg), dim3(g.waves * 64), (uint32_t)xq_bytes(a.cols), a);
     }
-    return c->launch(name + (xf ? "_xf" : ""), dim3(g.grid), dim3(g.waves * 64), (uint32_t)xq_bytes(a.cols), a);
+    return c->launch(name, dim3(g.grid), dim3(g.waves * 64), (uint32_t)xq_bytes(a.cols), a);
 }
 
 // x (times gamma) -> XQ with per-256 partial sums of x^2.
@@ -371,8 +382,24 @@ static ifr_status gemv_plain(ifr_ctx *c, float *out, const void *w, int32_t dtyp
     if (!c->gemv_exact) {
         // the GEMV kernel quantizes the f32 x into its LDS itself (the same
         // bytes as the quantize launch): one launch instead of two
-        const std::string one = std::string("gemv_") + p.fmt + "_plain_one_xf", loop = std::string("gemv_") + p.fmt + "_plain_xf";
-        if (allow_xf && cols % 16 == 0 && c->fn(one) && c->fn(loop)) return launch_gemv(c, p, "plain", a, 0, nullptr, true);
+        ifr_ctx::PlainXf &k = c->plain_xf[dtype];
+        if (!k.known) {
+            k.one = c->fn(std::string("gemv_") + p.fmt + "_plain_one_xf");
+            k.loop = c->fn(std::string("gemv_") + p.fmt + "_plain_xf");
+            k.known = true;
+        }
+        if (allow_xf && cols % 16 == 0 && k.one && k.loop) {
+            if (a.nb <= p.bpi && !c->gemv_waves && !c->gemv_max_grid && rows) { // as launch_gemv
+                const uint32_t g = (rows + GEMV_ONE_WAVES * 2 - 1) / (GEMV_ONE_WAVES * 2);
+                a.ks = 1;
+                a.nwaves = GEMV_ONE_WAVES;
+                return c->launch_fn(k.one, "gemv_plain_one_xf", dim3(g), dim3(GEMV_ONE_WAVES * 64), (uint32_t)xq_bytes(cols), a);
+            }
+            const IntGeom g = int_geom(c, p.bpi, "plain", a, 0);
+            a.ks = g.ks;
+            a.nwaves = g.waves;
+            return c->launch_fn(k.loop, "gemv_plain_xf", dim3(g.grid), dim3(g.waves * 64), (uint32_t)xq_bytes(cols), a);
+        }
         if (!xq) {
             if ((st = c->ensure_xq_scratch(xq_bytes(cols)))) return st;
             xq = (uint8_t *)c->xq_scratch;
@@ -953,7 +980,8 @@ IFR_API ifr_status ifr_create(int32_t device, const char *code_object_path, ifr_
     c->device = device;
     auto bail = [&](ifr_status st) {
         g_create_error = c->err;
-            if (c->module) hipModuleUnload(c->module);
+        if (c->ctl_host) hipHostFree(c->ctl_host);
+        if (c->module) hipModuleUnload(c->module);
         if (c->stream) hipStreamDestroy(c->stream);
         delete c;
         return st;
@@ -983,6 +1011,7 @@ IFR_API ifr_status ifr_create(int32_t device, const char *code_object_path, ifr_
         return bail(st);
     for (auto &e : c->events)
         if ((st = c->hip(hipEventCreate(&e), "hipEventCreate"))) return bail(st);
+    if ((st = c->hip(hipHostMalloc((void **)&c->ctl_host, sizeof(StepCtl), 0), "hipHostMalloc"))) return bail(st);
     if ((st = c->hip(ifr_noalloc_init(device, &c->noalloc_scratch), "hipGetSymbolAddress(scratch)"))) return bail(st);
     *out = c;
     return IFR_OK;
@@ -994,6 +1023,7 @@ IFR_API void ifr_destroy(ifr_ctx *c) {
     hipStreamSynchronize(c->stream);
     if (c->scratch) hipFree(c->scratch);
     if (c->xq_scratch) hipFree(c->xq_scratch);
+    if (c->ctl_host) hipHostFree(c->ctl_host);
     for (auto &e : c->events)
         if (e) hipEventDestroy(e);
     if (c->module) hipModuleUnload(c->module);
@@ -1690,6 +1720,23 @@ IFR_API ifr_status ifr_llama2_state_create(ifr_ctx *c, const ifr_llama2_config *
 
 IFR_API void ifr_llama2_state_destroy(ifr_llama2_state *s) { state_free(s); }
 
+// The state's control block and op parameters, set in one launch behind the
+// queued work (three blocking copies of a few bytes each took about 25 us).
+static ifr_status launch_set_pos(ifr_ctx *c, ifr_llama2_state *s, const StepCtl &ctl) {
+    const ifr_llama2_config &cfg = s->cfg;
+    SetPosArgs a{};
+    a.ctl = s->ctl;
+    a.rope = s->rope_cfg;
+    a.attn = s->attn_params;
+    a.ctl_v = ctl;
+    const ifr_rope_config rope{s->head_size, s->kv_dim, ctl.pos, cfg.rope_theta};
+    const ifr_attn_params ap{cfg.max_pos, s->kv_dim, s->kv_mul, cfg.n_heads, s->head_size, ctl.pos};
+    static_assert(sizeof rope == sizeof a.rope_v && sizeof ap == sizeof a.attn_v, "words of the parameter structs");
+    memcpy(a.rope_v, &rope, sizeof rope);
+    memcpy(a.attn_v, &ap, sizeof ap);
+    return c->launch("set_pos_k", dim3(1), dim3(64), 0, a);
+}
+
 IFR_API ifr_status ifr_llama2_state_reset(ifr_llama2_state *s, const uint32_t *prompt, uint32_t n, uint32_t pos) {
     if (!s) return IFR_EINVAL;
     ifr_ctx *c = s->ctx;
@@ -1700,15 +1747,12 @@ IFR_API ifr_status ifr_llama2_state_reset(ifr_llama2_state *s, const uint32_t *p
     for (uint32_t i = 0; i < n; i++)
         if (prompt[i] >= cfg.vocab) return c->fail(IFR_EINVAL, "prompt token %u out of range", prompt[i]);
     ifr_status st;
-    if ((st = c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize"))) return st;
-    if (n && (st = c->hip(hipMemcpy(s->tokens, prompt, n * 4, hipMemcpyHostToDevice), "hipMemcpy(tokens)"))) return st;
-    StepCtl ctl{pos, n, cfg.max_pos, 0};
+    if (n && (st = c->hip(hipMemcpyAsync(s->tokens, prompt, n * 4, hipMemcpyHostToDevice, c->stream), "hipMemcpyAsync(tokens)")))
+        return st;
     s->host_pos = pos;
-    ifr_rope_config rope{s->head_size, s->kv_dim, pos, cfg.rope_theta};
-    ifr_attn_params ap{cfg.max_pos, s->kv_dim, s->kv_mul, cfg.n_heads, s->head_size, pos};
-    if ((st = c->hip(hipMemcpy(s->ctl, &ctl, sizeof ctl, hipMemcpyHostToDevice), "hipMemcpy(ctl)"))) return st;
-    if ((st = c->hip(hipMemcpy(s->rope_cfg, &rope, sizeof rope, hipMemcpyHostToDevice), "hipMemcpy(rope)"))) return st;
-    return c->hip(hipMemcpy(s->attn_params, &ap, sizeof ap, hipMemcpyHostToDevice), "hipMemcpy(attn)");
+    if ((st = launch_set_pos(c, s, StepCtl{pos, n, cfg.max_pos, 0}))) return st;
+    // the prompt may be reused, and the state read in any way, from here on
+    return c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
 }
 
 static ifr_status check_weights(ifr_ctx *c, const ifr_llama2_state *s, const ifr_llama2_weights *w) {
@@ -1928,9 +1972,10 @@ IFR_API ifr_status ifr_llama2_prefill(ifr_ctx *c, ifr_llama2_state *s, const ifr
     if (!n) return IFR_OK;
     if ((st = pf_ensure_scratch(s))) return st;
     // the position lives on the device: read it once
-    StepCtl ctl;
-    if ((st = c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize"))) return st;
-    if ((st = c->hip(hipMemcpy(&ctl, s->ctl, sizeof ctl, hipMemcpyDeviceToHost), "hipMemcpy(ctl)"))) return st;
+    if ((st = c->hip(hipMemcpyAsync(c->ctl_host, s->ctl, sizeof(StepCtl), hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync(ctl)")) ||
+        (st = c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize")))
+        return st;
+    StepCtl ctl = *c->ctl_host;
     const uint32_t pos0 = ctl.pos;
     if ((uint64_t)pos0 + n > cfg.max_pos) return c->fail(IFR_EINVAL, "prefill: %u tokens from position %u exceed max_pos", n, pos0);
     if (pos0 + n > ctl.n_forced) return c->fail(IFR_EINVAL, "prefill: positions up to %u hold no prompt token", pos0 + n);
@@ -2023,15 +2068,10 @@ IFR_API ifr_status ifr_llama2_prefill(ifr_ctx *c, ifr_llama2_state *s, const ifr
         }
     }
     // advance the device position (and the unfused path's op parameters)
-    const uint32_t pos = pos0 + n;
-    if ((st = c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize"))) return st;
-    ctl.pos = pos;
-    s->host_pos = pos;
-    ifr_rope_config rope{hs, kvd, pos, cfg.rope_theta};
-    ifr_attn_params ap{cfg.max_pos, kvd, G, cfg.n_heads, hs, pos};
-    if ((st = c->hip(hipMemcpy(s->ctl, &ctl, sizeof ctl, hipMemcpyHostToDevice), "hipMemcpy(ctl)"))) return st;
-    if ((st = c->hip(hipMemcpy(s->rope_cfg, &rope, sizeof rope, hipMemcpyHostToDevice), "hipMemcpy(rope)"))) return st;
-    return c->hip(hipMemcpy(s->attn_params, &ap, sizeof ap, hipMemcpyHostToDevice), "hipMemcpy(attn)");
+    ctl.pos = pos0 + n;
+    s->host_pos = ctl.pos;
+    if ((st = launch_set_pos(c, s, ctl))) return st;
+    return c->hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
 }
 
 static void host_advance(ifr_llama2_state *s, uint32_t steps) {

@@ -210,6 +210,16 @@ struct EmbedArgs {
     uint32_t pad;
 };
 
+// Sets a state's position: its control block and the op parameter structs of
+// the one-op-per-kernel path, all given by value.
+struct SetPosArgs {
+    StepCtl *ctl;
+    void *rope; // ifr_rope_config
+    void *attn; // ifr_attn_params
+    StepCtl ctl_v;
+    uint32_t rope_v[4], attn_v[6];
+};
+
 // Quantizes an activation vector (XQ layout), optionally times gamma, with
 // per-workgroup partial sums of x^2.
 struct QActArgs {

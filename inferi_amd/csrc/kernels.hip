@@ -191,6 +191,7 @@ extern "C" __global__ void __launch_bounds__(256) sample_prob_k(SampleArgs a) { 
 extern "C" __global__ void __launch_bounds__(256) sample_group_k(SampleArgs a) { sample_group_body(a); }
 extern "C" __global__ void __launch_bounds__(1024) sample_select_k(SampleArgs a) { sample_select_body(a); }
 extern "C" __global__ void __launch_bounds__(256) quant_act_k(QActArgs a) { quant_act_body(a); }
+extern "C" __global__ void __launch_bounds__(64) set_pos_k(SetPosArgs a) { set_pos_body(a); }
 extern "C" __global__ void __launch_bounds__(256) kv_store_k(KvStoreArgs a) { kv_store_body(a); }
 extern "C" __global__ void __launch_bounds__(256) dequant_k(DequantArgs a) { dequant_body(a); }
 extern "C" __global__ void __launch_bounds__(64) quantize_k(QuantArgs a) { quantize_body(a); }
