@@ -66,30 +66,44 @@ IFR_DEV uint64_t smp_key(uint32_t bits, uint32_t i) { return ((uint64_t)bits << 
 IFR_DEV uint64_t key_fx(uint64_t key) { return prob_fx(__uint_as_float((uint32_t)(key >> 32))); }
 IFR_DEV uint32_t key_index(uint64_t key) { return 0xFFFFFFFFu - (uint32_t)key; }
 
-IFR_DEV uint64_t wave_sum_u64(uint64_t v) {
-    for (int sh = 32; sh >= 1; sh >>= 1) v += __shfl_xor(v, sh, 64);
-    return v;
+// One step of the scans below: v of the lane that `CTRL` names, or `id` in
+// lanes that have none or whose row is not in ROWS.
+template <int CTRL, int ROWS>
+IFR_DEV uint64_t smp_dpp(uint64_t v, uint64_t id) {
+    const uint32_t lo = __builtin_amdgcn_update_dpp((int)(uint32_t)id, (int)(uint32_t)v, CTRL, ROWS, 0xF, false);
+    const uint32_t hi =
+        __builtin_amdgcn_update_dpp((int)(uint32_t)(id >> 32), (int)(uint32_t)(v >> 32), CTRL, ROWS, 0xF, false);
+    return (uint64_t)hi << 32 | lo;
 }
+// Inclusive scan over the wave's 64 lanes (all of them active), id the
+// identity of op: within rows of 16 by shifts of 1, 2, 4, 8, then row 0's
+// total to row 1 and row 2's to row 3, then the lower half's to the upper.
+// DPP moves, because a step of a 64-bit scan by ds_bpermute is two LDS round
+// trips and sample_select is a chain of such scans.
+template <class Op>
+IFR_DEV uint64_t wave_scan_u64(uint64_t v, uint64_t id, Op op) {
+    v = op(v, smp_dpp<0x111, 0xF>(v, id));
+    v = op(v, smp_dpp<0x112, 0xF>(v, id));
+    v = op(v, smp_dpp<0x114, 0xF>(v, id));
+    v = op(v, smp_dpp<0x118, 0xF>(v, id));
+    v = op(v, smp_dpp<0x142, 0xA>(v, id));
+    return op(v, smp_dpp<0x143, 0xC>(v, id));
+}
+// Lane 63's value to every lane.
+IFR_DEV uint64_t wave_last_u64(uint64_t v) {
+    const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, 63);
+    const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), 63);
+    return (uint64_t)hi << 32 | lo;
+}
+IFR_DEV uint64_t wave_incl_scan_u64(uint64_t v) {
+    return wave_scan_u64(v, 0, [](uint64_t a, uint64_t b) { return a + b; });
+}
+IFR_DEV uint64_t wave_sum_u64(uint64_t v) { return wave_last_u64(wave_incl_scan_u64(v)); }
 IFR_DEV uint64_t wave_max_u64(uint64_t v) {
-    for (int sh = 32; sh >= 1; sh >>= 1) {
-        const uint64_t o = __shfl_xor(v, sh, 64);
-        v = o > v ? o : v;
-    }
-    return v;
+    return wave_last_u64(wave_scan_u64(v, 0, [](uint64_t a, uint64_t b) { return a > b ? a : b; }));
 }
 IFR_DEV uint64_t wave_min_u64(uint64_t v) {
-    for (int sh = 32; sh >= 1; sh >>= 1) {
-        const uint64_t o = __shfl_xor(v, sh, 64);
-        v = o < v ? o : v;
-    }
-    return v;
-}
-IFR_DEV uint64_t wave_incl_scan_u64(uint64_t v, uint32_t lane) {
-    for (uint32_t d = 1; d < 64; d <<= 1) {
-        const uint64_t o = __shfl_up(v, d, 64);
-        if (lane >= d) v += o;
-    }
-    return v;
+    return wave_last_u64(wave_scan_u64(v, ~0ull, [](uint64_t a, uint64_t b) { return a < b ? a : b; }));
 }
 
 // Four consecutive values from i (zero past n); v is 16-byte aligned.
@@ -342,24 +356,21 @@ IFR_DEV void sample_group_body(const SampleArgs &a) {
         ex += c8[q];
     }
     // this workgroup's candidates per bucket
+    uint32_t rank[8]; // among this workgroup's of its bucket
 #pragma unroll
     for (int q = 0; q < 8; q++)
-        if (ii[q] < n && pr[q] >= cutoff) atomicAdd(&lc[__float_as_uint(pr[q]) >> 20], 1u);
+        rank[q] = ii[q] < n && pr[q] >= cutoff ? atomicAdd(&lc[__float_as_uint(pr[q]) >> 20], 1u) : 0;
     __syncthreads();
-    // reserve a range per bucket; lc becomes the fill cursor
+    // reserve a range per bucket
     for (uint32_t b = tid; b < 2048; b += SMPG_THREADS)
-        if (lc[b]) {
-            off[b] += atomicAdd(&smpw_cur(a.work)[b], lc[b]);
-            lc[b] = 0;
-        }
+        if (lc[b]) off[b] += atomicAdd(&smpw_cur(a.work)[b], lc[b]);
     __syncthreads();
     uint64_t *keys = smpw_keys(a.work);
 #pragma unroll
     for (int q = 0; q < 8; q++)
         if (ii[q] < n && pr[q] >= cutoff) {
             const uint32_t u = __float_as_uint(pr[q]);
-            const uint32_t r = atomicAdd(&lc[u >> 20], 1u);
-            keys[off[u >> 20] + r] = smp_key(u, ii[q]);
+            keys[off[u >> 20] + rank[q]] = smp_key(u, ii[q]);
         }
 }
 
@@ -368,75 +379,108 @@ IFR_DEV void sample_group_body(const SampleArgs &a) {
 struct SmpLds {
     uint64_t h0[2048];            // level-0 histogram of candidate mass (bits 30..20)
     uint32_t c0[2048];            // level-0 candidate counts
-    uint64_t h[2048];             // finer levels: masses, then index counts
+    uint64_t h[2048];             // level-1 masses, then index counts
+    uint64_t h2[512];             // level-2 masses
     uint32_t cnt[512], mini[512]; // level 2: keys and smallest index per bucket
     uint64_t keys[SMP_CAP];       // the group being searched, when it fits
-    uint64_t wtot[SMP_WAVES];
     uint64_t wkey[SMP_WAVES];
-    int32_t win;
-    uint64_t win_excl;
+    struct { // of one search; two, so that a search need not wait for the last one's readers
+        uint64_t wtot[SMP_WAVES];
+        uint32_t wcnt[SMP_WAVES];
+        int32_t win;
+        uint32_t win_cnt;
+        uint64_t win_excl;
+    } s[2];
     uint32_t found_idx;
     uint32_t ctl_pos;
 };
 
-// Thread order is sequence order and thread t holds v.  Returns, to every
-// thread, the first thread whose inclusive prefix sum exceeds t (-1: none),
-// the prefix before it in excl and the sum of all in total.
-IFR_DEV int32_t block_first_exceeding(SmpLds &L, uint64_t v, uint64_t t, uint64_t &excl, uint64_t &total) {
+// The workgroup's state in sample_select: `turn` selects L.s, `held` is the
+// group whose keys are in L.keys.
+struct SmpCtx {
+    SmpLds &L;
+    uint32_t turn = 0;
+    const uint64_t *held = nullptr;
+};
+
+// A sequence of pairs in thread order: thread t holds elements 2t and 2t + 1,
+// v0 and v1.  Returns, to every thread, the first element whose inclusive
+// prefix sum exceeds t (-1: none), the prefix before it in excl, the sum of
+// all in total, and in cnt the sum of c0, c1 over the elements before it.
+// Two barriers, and nothing of the caller's is read after the second: the
+// arrays that v and c came from may be rewritten at once.  sample_select
+// runs as one workgroup, and its time is the chain of these searches and of
+// the passes over a group between them: at 128256 elements 19.8 us with
+// ds_bpermute scans, a third barrier, a search of its own for a group's start
+// and the group read twice, 16.5 us as it stands.  One loop over the levels
+// in place of a pass written out for each was smaller and took 21.9 us.
+IFR_DEV int32_t block_first_exceeding(SmpCtx &X, uint64_t v0, uint64_t v1, uint64_t t, uint64_t &excl, uint64_t &total,
+                                      uint32_t c0, uint32_t c1, uint32_t &cnt) {
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    uint64_t incl = wave_incl_scan_u64(v, lane);
-    if (lane == 63) L.wtot[wave] = incl;
-    if (tid == 0) L.win = -1;
+    auto &S = X.L.s[X.turn];
+    X.turn ^= 1;
+    uint64_t incl = wave_incl_scan_u64(v0 + v1);
+    const uint64_t ci = wave_incl_scan_u64(c0 + c1);
+    if (lane == 63) {
+        S.wtot[wave] = incl;
+        S.wcnt[wave] = (uint32_t)ci;
+    }
+    if (tid == 0) S.win = -1;
     __syncthreads();
     uint64_t base = 0, tot = 0;
+    uint32_t cb = 0;
+#pragma unroll
     for (uint32_t w = 0; w < SMP_WAVES; w++) {
-        const uint64_t s = L.wtot[w];
+        const uint64_t s = S.wtot[w];
         base += w < wave ? s : 0;
+        cb += w < wave ? S.wcnt[w] : 0;
         tot += s;
     }
     incl += base;
-    const uint64_t ex = incl - v;
+    const uint64_t ex = incl - (v0 + v1);
     if (ex <= t && t < incl) { // at most one thread: the intervals are disjoint
-        L.win = (int32_t)tid;
-        L.win_excl = ex;
+        const bool second = ex + v0 <= t;
+        S.win = (int32_t)(2 * tid + second);
+        S.win_excl = ex + (second ? v0 : 0);
+        S.win_cnt = cb + (uint32_t)ci - c1 - (second ? 0 : c0);
     }
     __syncthreads();
-    const int32_t w = L.win;
-    excl = L.win_excl;
+    excl = S.win_excl;
+    cnt = S.win_cnt;
     total = tot;
-    __syncthreads(); // L.win and L.wtot are rewritten by the next call
-    return w;
+    return S.win;
+}
+// The same of one element per thread.
+IFR_DEV int32_t block_first_exceeding(SmpCtx &X, uint64_t v, uint64_t t, uint64_t &excl, uint64_t &total) {
+    uint32_t cnt;
+    const int32_t e = block_first_exceeding(X, v, 0, t, excl, total, 0, 0, cnt);
+    return e < 0 ? e : e >> 1;
 }
 
 // Buckets h[0..nb) visited from the highest (desc) or the lowest: the first
 // whose running sum, starting at `above` (<= t), exceeds t.  Returns it (-1:
 // none) and leaves in `above` the sum before it (all of it when there is
-// none).  nb <= 2048.
-IFR_DEV int32_t smp_find_bucket(SmpLds &L, const uint64_t *h, uint32_t nb, uint64_t &above, uint64_t t,
-                                bool desc = true) {
+// none), and in off, given the buckets' counts c, the sum of those before it.
+// nb <= 2048.
+IFR_DEV int32_t smp_find_bucket(SmpCtx &X, const uint64_t *h, uint32_t nb, uint64_t &above, uint64_t t,
+                                bool desc = true, const uint32_t *c = nullptr, uint32_t *off = nullptr) {
     auto at = [&](uint32_t d) { return desc ? nb - 1 - d : d; };
     const uint32_t d0 = 2 * threadIdx.x, d1 = d0 + 1;
     const uint64_t a0 = d0 < nb ? h[at(d0)] : 0, a1 = d1 < nb ? h[at(d1)] : 0;
+    const uint32_t c0 = c && d0 < nb ? c[at(d0)] : 0, c1 = c && d1 < nb ? c[at(d1)] : 0;
     uint64_t ex, total;
-    const int32_t w = block_first_exceeding(L, a0 + a1, t - above, ex, total);
-    if (w < 0) {
-        above += total;
-        return -1;
-    }
-    const uint32_t e0 = 2 * (uint32_t)w;
-    const uint64_t m0 = h[at(e0)];
-    if (ex + m0 > t - above) {
-        above += ex;
-        return (int32_t)at(e0);
-    }
-    above += ex + m0;
-    return (int32_t)at(e0 + 1);
+    uint32_t before;
+    const int32_t e = block_first_exceeding(X, a0, a1, t - above, ex, total, c0, c1, before);
+    above += e < 0 ? total : ex;
+    if (e < 0) return -1;
+    if (off) *off = before;
+    return (int32_t)at((uint32_t)e);
 }
 
 // Sum over the workgroup of one value per thread (every thread gets it).
-IFR_DEV uint64_t smp_block_sum(SmpLds &L, uint64_t v) {
+IFR_DEV uint64_t smp_block_sum(SmpCtx &X, uint64_t v) {
     uint64_t ex, total;
-    block_first_exceeding(L, v, ~0ull, ex, total);
+    block_first_exceeding(X, v, ~0ull, ex, total);
     return total;
 }
 
@@ -453,7 +497,7 @@ IFR_DEV uint32_t smp_locate(SmpLds &L, const float *p, uint32_t n, uint32_t c, u
 #pragma unroll
         for (int k = 0; k < 4; k++) w[k] = i0 + k < n ? wt(x[k], i0 + k) : 0;
         const uint64_t s = w[0] + w[1] + w[2] + w[3];
-        const uint64_t incl = wave_incl_scan_u64(s, lane);
+        const uint64_t incl = wave_incl_scan_u64(s);
         const uint64_t ex = incl - s;
         const bool hit = ex <= t && t < incl;
         if (__ballot(hit) == 0) {
@@ -479,18 +523,19 @@ IFR_DEV uint32_t smp_locate(SmpLds &L, const float *p, uint32_t n, uint32_t c, u
     return r;
 }
 
-// Copies the group seg[0..C) into L.keys when it fits.
-IFR_DEV void smp_seg_load(SmpLds &L, const uint64_t *seg, uint32_t C) {
-    if (C > SMP_CAP) return;
+// Copies the group seg[0..C) into L.keys when it fits and is not there.
+// The caller's next barrier publishes it.
+IFR_DEV void smp_seg_load(SmpCtx &X, const uint64_t *seg, uint32_t C) {
+    if (C > SMP_CAP || X.held == seg) return;
+    X.held = seg;
     for (uint32_t e = threadIdx.x; e < C; e += 4 * SMP_THREADS) {
         uint64_t k[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) k[j] = seg[min(e + j * SMP_THREADS, C - 1)];
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            if (e + j * SMP_THREADS < C) L.keys[e + j * SMP_THREADS] = k[j];
+            if (e + j * SMP_THREADS < C) X.L.keys[e + j * SMP_THREADS] = k[j];
     }
-    __syncthreads();
 }
 
 // Calls f(key) for every key of the group seg[0..C): from L.keys when it was
@@ -517,37 +562,37 @@ IFR_DEV void smp_seg_for(const SmpLds &L, const uint64_t *seg, uint32_t C, F &&f
 // buckets), first exceeds t, counting only keys >= bound (the list up to
 // and including the key `bound`; 0: all).  Returns its key (0 if none; the
 // callers pass a group that holds the crossing) and the running mass there.
-IFR_DEV uint64_t smp_select_group(SmpLds &L, const uint64_t *seg, uint32_t C, uint32_t b0, uint64_t above, uint64_t t,
+IFR_DEV uint64_t smp_select_group(SmpCtx &X, const uint64_t *seg, uint32_t C, uint32_t b0, uint64_t above, uint64_t t,
                                   uint64_t bound, uint64_t &cum) {
     const uint32_t tid = threadIdx.x;
-    smp_seg_load(L, seg, C);
+    SmpLds &L = X.L;
+    smp_seg_load(X, seg, C);
     // level 1: bits 19..9
     for (uint32_t b = tid; b < 2048; b += SMP_THREADS) L.h[b] = 0;
-    __syncthreads();
-    smp_seg_for(L, seg, C, [&](uint64_t key) {
-        if (key >= bound) atomicAdd(&L.h[(uint32_t)(key >> 41) & 0x7FFu], (unsigned long long)key_fx(key));
-    });
-    __syncthreads();
-    const int32_t b1 = smp_find_bucket(L, L.h, 2048, above, t);
-    if (b1 < 0) return 0;
-    // level 2: bits 8..0, with key counts and the smallest index
     for (uint32_t b = tid; b < 512; b += SMP_THREADS) {
-        L.h[b] = 0;
+        L.h2[b] = 0;
         L.cnt[b] = 0;
         L.mini[b] = 0xFFFFFFFFu;
     }
     __syncthreads();
     smp_seg_for(L, seg, C, [&](uint64_t key) {
+        if (key >= bound) atomicAdd(&L.h[(uint32_t)(key >> 41) & 0x7FFu], (unsigned long long)key_fx(key));
+    });
+    __syncthreads();
+    const int32_t b1 = smp_find_bucket(X, L.h, 2048, above, t);
+    if (b1 < 0) return 0;
+    // level 2: bits 8..0, with key counts and the smallest index
+    smp_seg_for(L, seg, C, [&](uint64_t key) {
         const uint32_t u = (uint32_t)(key >> 32);
         if (key >= bound && ((u >> 9) & 0x7FFu) == (uint32_t)b1) {
             const uint32_t d = u & 0x1FFu;
-            atomicAdd(&L.h[d], (unsigned long long)key_fx(key));
+            atomicAdd(&L.h2[d], (unsigned long long)key_fx(key));
             atomicAdd(&L.cnt[d], 1u);
             atomicMin(&L.mini[d], key_index(key));
         }
     });
     __syncthreads();
-    const int32_t b2 = smp_find_bucket(L, L.h, 512, above, t);
+    const int32_t b2 = smp_find_bucket(X, L.h2, 512, above, t);
     if (b2 < 0) return 0;
     const uint32_t v = (b0 << 20) | ((uint32_t)b1 << 9) | (uint32_t)b2;
     const uint64_t w = prob_fx(__uint_as_float(v));
@@ -570,7 +615,7 @@ IFR_DEV uint64_t smp_select_group(SmpLds &L, const uint64_t *seg, uint32_t C, ui
                     atomicAdd(&L.h[lvl == 0 ? i >> 9 : i & 0x1FFu], 1ull);
             });
             __syncthreads();
-            (lvl == 0 ? ia : ib) = smp_find_bucket(L, L.h, 512, below, k, false);
+            (lvl == 0 ? ia : ib) = smp_find_bucket(X, L.h, 512, below, k, false);
             if ((lvl == 0 ? ia : ib) < 0) return 0;
         }
         idx = ((uint32_t)ia << 9) | (uint32_t)ib;
@@ -581,6 +626,7 @@ IFR_DEV uint64_t smp_select_group(SmpLds &L, const uint64_t *seg, uint32_t C, ui
 
 IFR_DEV void sample_select_body(const SampleArgs &a) {
     __shared__ SmpLds L;
+    SmpCtx X{L};
     const uint32_t tid = threadIdx.x;
 
     const uint32_t n = a.n, nch = (n + SMP_CHUNK - 1) / SMP_CHUNK;
@@ -622,18 +668,14 @@ IFR_DEV void sample_select_body(const SampleArgs &a) {
         // the coin, n - 1 if none does
         const uint64_t cfx = prob_fx(coin);
         uint64_t ex, total;
-        const int32_t c = block_first_exceeding(L, cm, cfx, ex, total);
+        const int32_t c = block_first_exceeding(X, cm, cfx, ex, total);
         idx = c < 0 ? n - 1
                     : smp_locate(L, a.probs, n, (uint32_t)c, cfx - ex, n - 1,
                                  [](float x, uint32_t) -> uint64_t { return prob_fx(x); });
     } else {
         const uint64_t *keys = smpw_keys(a.work);
-        // the group of bucket b starts after the candidates of higher buckets
-        auto group = [&](int32_t b) {
-            uint64_t v = 0;
-            for (uint32_t q = (uint32_t)b + 1 + 2 * tid; q < (uint32_t)b + 3 + 2 * tid; q++) v += q < 2048 ? L.c0[q] : 0;
-            return keys + smp_block_sum(L, v);
-        };
+        // a bucket's group starts after the candidates of higher buckets
+        uint32_t off = 0;
         if (n0 == 0) {
             // no probability reaches the cutoff: the reference's sample_topp
             // has nothing to sort and fails; take the most probable token
@@ -644,14 +686,13 @@ IFR_DEV void sample_select_body(const SampleArgs &a) {
             // candidate, kmin) ...
             const uint64_t tfx = prob_fx(a.topp);
             uint64_t above1 = 0;
-            const int32_t b1 = smp_find_bucket(L, L.h0, 2048, above1, tfx);
+            const int32_t b1 = smp_find_bucket(X, L.h0, 2048, above1, tfx, true, L.c0, &off);
             uint64_t lkey = kmin, cum = above1;
             if (b1 >= 0) {
-                const uint64_t *g = group(b1);
-                lkey = smp_select_group(L, g, L.c0[b1], (uint32_t)b1, above1, tfx, 0, cum);
+                lkey = smp_select_group(X, keys + off, L.c0[b1], (uint32_t)b1, above1, tfx, 0, cum);
                 if (!lkey) { // cannot happen: the bucket holds the crossing
                     lkey = kmin;
-                    cum = smp_block_sum(L, L.h0[2 * tid] + L.h0[2 * tid + 1]);
+                    cum = smp_block_sum(X, L.h0[2 * tid] + L.h0[2 * tid + 1]);
                 }
             }
             // ... then the first element of the truncated list whose running
@@ -664,12 +705,11 @@ IFR_DEV void sample_select_body(const SampleArgs &a) {
             }
             __syncthreads();
             uint64_t above2 = 0;
-            const int32_t b2 = smp_find_bucket(L, L.h0, 2048, above2, rfx);
+            const int32_t b2 = smp_find_bucket(X, L.h0, 2048, above2, rfx, true, L.c0, &off);
             idx = key_index(lkey);
             if (b2 >= 0) {
-                const uint64_t *g = group(b2);
                 uint64_t c2;
-                const uint64_t key2 = smp_select_group(L, g, L.c0[b2], (uint32_t)b2, above2, rfx, lkey, c2);
+                const uint64_t key2 = smp_select_group(X, keys + off, L.c0[b2], (uint32_t)b2, above2, rfx, lkey, c2);
                 if (key2) idx = key_index(key2);
             }
         }

@@ -255,3 +255,17 @@ def test_set_sampler_rejects(ctx):
     finally:
         s.close()
         w.close()
+
+
+@pytest.mark.parametrize("c", [1, 2, 8191, 8192, 8193])
+def test_sample_topp_group_sizes(ctx, oracle_lib, c):
+    """A crossing group of c distinct probabilities, on both sides of the
+    8192 keys that stay in LDS from the truncation's search to the choice's,
+    between groups of a few higher and many lower ones."""
+    rng = np.random.default_rng(c)
+    x = np.full(40000, -9.0, np.float32)
+    x[:c] = (np.arange(c) * (0.05 / c)).astype(np.float32)  # within one bucket or two neighbours
+    x[c : c + 3] = 0.5
+    x = x[rng.permutation(x.size)]
+    for topp in (0.3, 0.9):
+        check_case(ctx, x, 1.0, topp, COINS)
