@@ -164,6 +164,10 @@ def lib() -> C.CDLL:
 
 
 def row_bytes(dtype: int, cols: int) -> int:
+    """Bytes of one row; cols is a whole number of blocks (rounded down, a
+    buffer sized by it would be short of what ``quantize`` writes)."""
+    if cols % BLOCK_ELEMS[dtype]:
+        raise ValueError(f"{cols} columns are not whole blocks of {BLOCK_ELEMS[dtype]}")
     return cols // BLOCK_ELEMS[dtype] * BLOCK_BYTES[dtype]
 
 

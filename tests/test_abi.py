@@ -68,3 +68,14 @@ def test_product_never_uses_the_oracle():
             if f.endswith((".py", ".cpp", ".h", ".hip")):
                 text = open(os.path.join(dirpath, f)).read()
                 assert "import oracle" not in text and "liboracle" not in text and "oracle.h" not in text, f
+
+
+def test_row_bytes_takes_whole_blocks_only():
+    """Rounded down, a row of 5504 columns would get 21 of its 21.5 Q4_K
+    blocks, and quantizing the matrix would write past its buffer."""
+    import inferi_amd as I
+
+    assert I.row_bytes(I.Q4_K, 5632) == 22 * 144 and I.row_bytes(I.F32, 5) == 20
+    for dtype, cols in ((I.Q4_K, 5504), (I.Q8_0, 48), (I.Q6_K, 896)):
+        with pytest.raises(ValueError):
+            I.row_bytes(dtype, cols)
