@@ -423,16 +423,27 @@ static uint32_t attn_splits_for(uint32_t T, uint32_t head_size) {
     return std::max(1u, std::min(ATTN_SPLITS_MAX, (uint32_t)(((uint64_t)T + q - 1) / q)));
 }
 // A KV head's query heads go to n_sub workgroups of gt heads each (the last
-// one holding the rest): gt at most 4 while the positions' K and V rows are
-// under 8 MB, else at most 8.  A group's heads share one pass over the rows
-// but wait for each other's arithmetic; below that size the rows' second read
-// comes from the L2 (us for split and merge, 8 or 4 heads at most: 32 heads
-// over 4 of 64 dims, f16, 1 MB 10.4 and 7.7, 4 MB 10.4 and 8.4; 12 over 2 of
-// 128, f32, 4 MB 9.8 and 9.1, 17 MB 12.3 and 13.9; 40 over 8 of 128, f16, 4 MB
-// 8.7 and 8.3, 8.4 MB 9.5 and 10.3).
-static void attn_groups(uint32_t kv_mul, uint64_t kv_bytes, uint32_t &n_sub, uint32_t &gt) {
-    const uint32_t most = kv_bytes < 8000000 ? 4 : ATTN_GT_MAX;
-    n_sub = (kv_mul + most - 1) / most;
+// one holding the rest): at most 8 heads, or at most 4 where that is faster.  A
+// group's heads share one pass over the rows but wait for each other's
+// arithmetic; smaller groups read the rows again, from the L2, and add
+// workgroups.  They are taken while the launch still fits the chip at one
+// workgroup per CU; past that only with f16 rows (half the bytes to read again),
+// where the larger groups take as many rounds of the chip anyway or hold 7 or 8
+// heads, and never from 8 MB of rows on.  us for split and merge, 8 or 4 heads
+// at most, caches from memory: 32 heads over 4 of 64, f16, 4 MB (240 workgroups
+// of 4) 10.8 and 8.7; 12 over 2 of 128, f32, 7.8 MB (240) 10.5 and 9.8; 24 over 2
+// of 128, f32, 4 MB (186) 10.8 and 10.2, 6 MB (276) 11.1 and 12.6; 20 over 2 of
+// 80, f16, 2 MB (294) 9.4 and 10.5; 40 over 8 of 128, f16, 7.8 MB (480) 9.6 and
+// 9.8; 32 over 4 of 128, f16, 7.8 MB (480) 11.5 and 10.4; 24 over 2 of 128, f16, 5
+// MB (462, and 308 of the larger) 11.8 and 10.6.
+static void attn_groups(uint32_t n_cu, uint32_t n_kv, uint32_t kv_mul, uint32_t n_splits, uint64_t kv_bytes, bool f16,
+                        uint32_t &n_sub, uint32_t &gt) {
+    const uint32_t n8 = (kv_mul + ATTN_GT_MAX - 1) / ATTN_GT_MAX, n4 = (kv_mul + 3) / 4;
+    const uint64_t w4 = (uint64_t)n_kv * n_splits * n4, w8 = (uint64_t)n_kv * n_splits * n8;
+    auto rounds = [&](uint64_t w) { return (w + n_cu - 1) / n_cu; };
+    const bool eight = (kv_mul + n8 - 1) / n8 == 8 || kv_mul == 7;
+    const bool four = kv_bytes < 8000000 && (w4 <= n_cu || (f16 && (rounds(w4) <= rounds(w8) || eight)));
+    n_sub = four ? n4 : n8;
     gt = (kv_mul + n_sub - 1) / n_sub;
 }
 
@@ -461,17 +472,19 @@ constexpr uint32_t ATTN_ONE_ELEMS = 65536;
 // head_size, kv_mul, n_splits, spec_rows and n_out; n_sub is set here.
 static ifr_status launch_attn(ifr_ctx *c, int32_t kv_dtype, AttnArgs &a, uint32_t n_kv_heads) {
     char name[64];
-    const char *kv = kv_dtype == IFR_F16 ? "f16" : "f32";
+    const bool f16 = kv_dtype == IFR_F16;
+    const char *kv = f16 ? "f16" : "f32";
     const uint32_t hsp = attn_hsp(a.head_size);
     if (a.head_size % 16 == 0 && (uint64_t)a.spec_rows * hsp <= ATTN_ONE_ELEMS) {
         // as many waves as one batch of the positions takes (4 or, f32, 2 per lane)
-        const uint32_t per_wave = 64 / (hsp / 8) * (kv_dtype == IFR_F16 ? 4u : 2u);
+        const uint32_t per_wave = 64 / (hsp / 8) * (f16 ? 4u : 2u);
         const uint32_t nw = std::min(ATTN_ONE_WAVES, std::max(4u, (a.spec_rows + per_wave - 1) / per_wave));
         snprintf(name, sizeof name, "attn_one_%s_h%u", kv, hsp);
         return c->launch(name, dim3(n_kv_heads * a.kv_mul), dim3(nw * 64), 0, a);
     }
     uint32_t n_sub, gt;
-    attn_groups(a.kv_mul, (uint64_t)a.spec_rows * a.kv_dim * (kv_dtype == IFR_F16 ? 4 : 8), n_sub, gt);
+    attn_groups((uint32_t)c->n_cu, n_kv_heads, a.kv_mul, a.n_splits,
+                (uint64_t)a.spec_rows * a.kv_dim * (f16 ? 4 : 8), f16, n_sub, gt);
     a.n_sub = n_sub;
     snprintf(name, sizeof name, "attn_%s_h%u_g%u", kv, hsp, gt);
     ifr_status st = c->launch(name, dim3(n_kv_heads * n_sub, a.n_splits), dim3(256), 0, a);

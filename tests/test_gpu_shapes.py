@@ -27,9 +27,9 @@ from tests.test_gpu_ops import _attn_case
 
 pytestmark = pytest.mark.gpu
 
-# (n_heads, n_kv_heads, head_size): group sizes 7, 6, 7, 3, 5, 12 (two
-# workgroups of 6), 32 (four of 8), 64, 10, 4, 4, 4, 2, 1 and head sizes 64,
-# 128, 32, 80, 96, 112, 40, 8
+# (n_heads, n_kv_heads, head_size): group sizes 7, 6, 7, 3, 5, 12, 32, 64, 10,
+# 4, 4, 4, 2, 1 (past 4, the split kernel's workgroups hold up to four heads
+# at these lengths) and head sizes 64, 128, 32, 80, 96, 112, 40, 8
 SHAPES = [(14, 2, 64), (12, 2, 128), (28, 4, 128), (24, 8, 128), (40, 8, 128), (24, 2, 128), (32, 1, 64),
           (64, 1, 32), (20, 2, 80), (16, 4, 96), (8, 2, 112), (16, 4, 32), (6, 3, 40), (4, 4, 8)]
 
@@ -124,7 +124,7 @@ MODELS = {
     # head size 80, 32 over 8
     "hs80": (dict(n_layers=2, hidden=2560, ffn=6912, n_heads=32, n_kv_heads=8, vocab=1500,
                   rope_theta=10000.0, rms_eps=1e-5), "Q4_K", False),
-    # 24 query heads of 32 over 2 KV heads (two workgroups of 6 per KV head)
+    # 24 query heads of 32 over 2 KV heads
     "g12_hs32": (dict(n_layers=2, hidden=768, ffn=2048, n_heads=24, n_kv_heads=2, vocab=1500,
                       rope_theta=10000.0, rms_eps=1e-5), "Q8_0", False),
 }
@@ -312,3 +312,37 @@ def test_attention_one_kernel_edges(ctx, oracle_lib, kv_f16, nh, nkv, hs):
     for T in (2, 31, 32, 33, 129, 256, 257, top - 1, top, top + 1):
         got, ref = _attn_case(ctx, nh, nkv, hs, top + 1, T - 1, kv_f16, rng)
         assert np.abs(got - ref).max() <= 1e-5, f"{T} positions"
+
+
+def _split_group(n_cu, nh, nkv, hs, T, f16):
+    """Query heads per workgroup of the split kernel for T positions, by the
+    launch's rule."""
+    kv_mul, hsp = nh // nkv, 64 if hs <= 64 else 128
+    S = max(1, min(256, -(-T // (8192 // hsp))))
+    n8, n4 = -(-kv_mul // 8), -(-kv_mul // 4)
+    r4, r8 = -(-nkv * S * n4 // n_cu), -(-nkv * S * n8 // n_cu)
+    eight = -(-kv_mul // n8) == 8 or kv_mul == 7
+    four = T * nkv * hs * (4 if f16 else 8) < 8000000 and (r4 <= 1 or (f16 and (r4 <= r8 or eight)))
+    return -(-kv_mul // (n4 if four else n8))
+
+
+@pytest.mark.parametrize("kv_f16", [True, False], ids=["f16", "f32"])
+@pytest.mark.parametrize("nh,nkv,hs", [(40, 8, 64), (48, 8, 64), (56, 8, 64), (64, 8, 64), (40, 8, 128), (48, 8, 128),
+                                       (56, 8, 128), (64, 8, 128), (24, 2, 128), (32, 2, 128), (20, 2, 80), (12, 1, 64)])
+def test_attention_split_group_edges(ctx, oracle_lib, kv_f16, nh, nkv, hs):
+    """The split kernel with at most four query heads per workgroup and with
+    five to eight, on both sides of each context where the launch changes
+    between them, for every group size, padded head size and cache type.  The
+    outputs are averages of N(0, 1) values: scores of N(0, 1) in f32 are off by
+    1e-6 at most, and so, relatively, are their weights and the outputs; 1e-5
+    allows ten times that."""
+    n_cu = ctx.device_info()[1]
+    rng = np.random.default_rng(nh * 100 + hs)
+    lo = 65536 // (64 if hs <= 64 else 128) + 1
+    gt = {T: _split_group(n_cu, nh, nkv, hs, T, kv_f16) for T in range(lo, 12000)}
+    edges = [T for T in range(lo, 11999) if gt[T] != gt[T + 1]][:3]
+    assert edges and max(gt[T + d] for T in edges for d in (0, 1)) > 4
+    for T in edges:
+        for n in (T, T + 1):
+            got, ref = _attn_case(ctx, nh, nkv, hs, n, n - 1, kv_f16, rng)
+            assert np.abs(got - ref).max() <= 1e-5, f"{n} positions, {gt[n]} heads"
