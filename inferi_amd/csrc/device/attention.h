@@ -436,9 +436,11 @@ __device__ inline void attn_merge_body(const AttnArgs &a) {
 // across lanes, the waves through LDS with one barrier.
 //
 // What bounds it: one memory round trip (about 2 us behind the launch) and
-// then one CU's share of the cache bandwidth (T x 512 bytes a workgroup with
-// f16 and 128 dims), so that it loses to the split kernel and its merge as T
-// grows; the host's rule and both sides' times are at launch_attn.
+// then what one CU draws (T x 512 bytes a workgroup with f16 and 128 dims), so
+// that it loses to the split kernel and its merge as T grows, and sooner where
+// no other head's workgroup brings the rows into the L2 (32 heads over 32 of
+// 64, f32, 900 positions, rows from memory: 15.0 us where split and merge take
+// 10.5); the host's rule and both sides' times are at attn_one_fits.
 template <bool F16>
 constexpr int ATTN_ONE_U = F16 ? 4 : 2;
 

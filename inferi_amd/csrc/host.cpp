@@ -456,16 +456,31 @@ static uint32_t attn_spec_for(uint32_t pos, uint32_t max_pos) {
     return (uint32_t)std::min<uint64_t>(max_pos, ((uint64_t)pos / ATTN_BUCKET + 1) * ATTN_BUCKET);
 }
 
-// Contexts this short (spec_rows x head size padded to 64 or 128) run in one
-// kernel, a workgroup per query head (device/attention.h attn_one_body):
-// up to 1024 positions of 64 dims, 512 of 128.  Past them one CU's pass over
-// its head's rows takes longer than the split kernel with its merge (us, one
-// kernel and split + merge: 32 heads over 8 of 128, f16, 145 positions 4.5
-// and 7.7, 512 6.6 and 7.7, 778 9.6 and 7.9; 32 over 4 of 64, f16, 145 3.9
-// and 7.7, 1024 6.5 and 7.7, 2048 9.7 and 7.9; 14 over 2 of 64, f32, 1024 8.6
-// and 9.0; 12 over 2 of 128, f32, 512 8.9 and 8.8).  Its output is quantized
-// in 16-value groups of one head, so the head size is a multiple of 16.
-constexpr uint32_t ATTN_ONE_ELEMS = 65536;
+// Short contexts run in one kernel, a workgroup per query head
+// (device/attention.h attn_one_body), instead of the split kernel and its merge:
+// up to 256 positions of 64 dims (elems = spec_rows x the head size padded to 64
+// or 128); up to 512 of 64 or 256 of 128 if two query heads or more share a KV
+// head's rows (which then come from the L2) or a layer's cache is small (kv_elems
+// = spec_rows x kv_dim); and up to 1024 of 64 or 512 of 128 if the rows are f16
+// and six heads share them.  Past these lines one CU's pass over rows that come
+// from memory takes longer than the split kernel with its merge.  (In a decode
+// step they do come from memory: the whole model is read between two uses of a
+// layer's cache.  Rows still in the L2 keep the one kernel ahead to 1024 of 64.)
+// us per layer of whole models' steps, split and one kernel, near the first and
+// near the last position of the bucket: 16 heads over 16 of 64, f16, to 256
+// 27.8 and 25.7, 27.8 and 25.7, to 512 28.8 and 29.1, 28.7 and 29.0; f32, to 512
+// 30.7 and 29.5, 30.6 and 31.3; 12 over 12 of 64, f32, to 512 26.8 and 24.2, 26.8
+// and 25.1; 32 over 8 of 64, f16, to 512 35.2 and 33.6, 35.2 and 33.6, to 768 35.3
+// and 34.9, 35.2 and 35.5; f32, to 512 36.7 and 34.1, 36.7 and 35.4, to 768 36.7
+// and 37.2, 36.7 and 38.5; 32 over 8 of 128, f16, to 512 48.2 and 47.7, 48.1 and
+// 48.5; 14 over 2 of 64, f16, to 1024 32.4 and 31.9, 32.4 and 32.2; 28 over 4 of
+// 128, f16, to 512 46.2 and 45.3, 46.1 and 46.2.  Its output is quantized in
+// 16-value groups of one head, so the head size is a multiple of 16.
+static bool attn_one_fits(uint32_t head_size, uint32_t kv_mul, uint64_t elems, uint64_t kv_elems, bool f16) {
+    if (head_size % 16 || elems > 65536) return false;
+    if (elems > 32768) return f16 && kv_mul >= 6;
+    return elems <= 16384 || kv_mul >= 2 || kv_elems < 500000;
+}
 
 // Attention of one token over the cache: the one-kernel form, or the split
 // pass over the sequence and the merge of its partials.  `a` carries
@@ -475,7 +490,8 @@ static ifr_status launch_attn(ifr_ctx *c, int32_t kv_dtype, AttnArgs &a, uint32_
     const bool f16 = kv_dtype == IFR_F16;
     const char *kv = f16 ? "f16" : "f32";
     const uint32_t hsp = attn_hsp(a.head_size);
-    if (a.head_size % 16 == 0 && (uint64_t)a.spec_rows * hsp <= ATTN_ONE_ELEMS) {
+    const uint64_t kv_elems = (uint64_t)a.spec_rows * a.kv_dim;
+    if (attn_one_fits(a.head_size, a.kv_mul, (uint64_t)a.spec_rows * hsp, kv_elems, f16)) {
         // as many waves as one batch of the positions takes (4 or, f32, 2 per lane)
         const uint32_t per_wave = 64 / (hsp / 8) * (f16 ? 4u : 2u);
         const uint32_t nw = std::min(ATTN_ONE_WAVES, std::max(4u, (a.spec_rows + per_wave - 1) / per_wave));
@@ -483,8 +499,7 @@ static ifr_status launch_attn(ifr_ctx *c, int32_t kv_dtype, AttnArgs &a, uint32_
         return c->launch(name, dim3(n_kv_heads * a.kv_mul), dim3(nw * 64), 0, a);
     }
     uint32_t n_sub, gt;
-    attn_groups((uint32_t)c->n_cu, n_kv_heads, a.kv_mul, a.n_splits,
-                (uint64_t)a.spec_rows * a.kv_dim * (f16 ? 4 : 8), f16, n_sub, gt);
+    attn_groups((uint32_t)c->n_cu, n_kv_heads, a.kv_mul, a.n_splits, kv_elems * (f16 ? 4 : 8), f16, n_sub, gt);
     a.n_sub = n_sub;
     snprintf(name, sizeof name, "attn_%s_h%u_g%u", kv, hsp, gt);
     ifr_status st = c->launch(name, dim3(n_kv_heads * n_sub, a.n_splits), dim3(256), 0, a);

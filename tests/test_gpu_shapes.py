@@ -244,9 +244,10 @@ def test_decode_position_buckets(ctx, oracle_lib):
     expects (the graph is captured again when the position leaves it).  A
     20,000-position cache decoded from position 240 across the 256 and 512
     bucket edges, with the graph and without; then the device position moved
-    past the host's bucket behind its back (the kernel's fallback to chunks
-    computed from the position it reads).  Logits against the oracle over
-    the same planted cache rows."""
+    past the host's bucket behind its back (the split kernel's fallback to
+    chunks computed from the position it reads).  Positions up to 511 take
+    the one-kernel attention, later ones the split one.  Logits against the
+    oracle over the same planted cache rows."""
     import inferi_amd as I
 
     cfg = I.Llama2Config(n_layers=2, hidden=256, ffn=512, n_heads=4, n_kv_heads=1, vocab=1000, max_pos=20000,
@@ -301,10 +302,10 @@ def test_decode_position_buckets(ctx, oracle_lib):
 @pytest.mark.parametrize("kv_f16", [True, False], ids=["f16", "f32"])
 @pytest.mark.parametrize("nh,nkv,hs", [(7, 1, 16), (6, 2, 48), (14, 2, 64), (10, 2, 80), (8, 8, 112), (40, 8, 128)])
 def test_attention_one_kernel_edges(ctx, oracle_lib, kv_f16, nh, nkv, hs):
-    """The one-kernel form at the edges of its waves and batches, on both
-    sides of the context where the split kernel takes over (1024 positions of
-    up to 64 dims, 512 of up to 128), with head sizes short of the padding,
-    and the split kernel's sub-groups of at most four heads past it.  The
+    """Short contexts at the edges of the one-kernel form's waves and batches,
+    with head sizes short of the padding, up to the longest it is taken for
+    (1024 positions of up to 64 dims, 512 of up to 128; the split kernel's
+    where the shape's line lies lower) and one past it.  The
     outputs are averages of at most 1025 N(0, 1) values in f32: 1e-5 leaves
     twenty times the largest difference two summation orders show."""
     rng = np.random.default_rng(nh * 100 + hs)
@@ -346,3 +347,70 @@ def test_attention_split_group_edges(ctx, oracle_lib, kv_f16, nh, nkv, hs):
         for n in (T, T + 1):
             got, ref = _attn_case(ctx, nh, nkv, hs, n, n - 1, kv_f16, rng)
             assert np.abs(got - ref).max() <= 1e-5, f"{n} positions, {gt[n]} heads"
+
+
+def _one_kernel(nh, nkv, hs, T, f16):
+    """Whether T positions run in the one-kernel form, by the launch's rule."""
+    kv_mul, elems = nh // nkv, T * (64 if hs <= 64 else 128)
+    if hs % 16 or elems > 65536:
+        return False
+    if elems > 32768:
+        return f16 and kv_mul >= 6
+    return elems <= 16384 or kv_mul >= 2 or T * nkv * hs < 500000
+
+
+@pytest.mark.parametrize("kv_f16", [True, False], ids=["f16", "f32"])
+@pytest.mark.parametrize("nh,nkv,hs", [(4, 4, 24), (8, 8, 64), (16, 16, 64), (32, 32, 64), (8, 4, 64), (14, 2, 64),
+                                       (16, 16, 80), (16, 16, 128), (32, 32, 128), (8, 2, 112), (12, 2, 128)])
+def test_attention_one_kernel_lines(ctx, oracle_lib, kv_f16, nh, nkv, hs):
+    """Both sides of the line between the one-kernel form and the split one,
+    wherever the shape's cache type, sharing and size put it.  The bound as in
+    test_attention_one_kernel_edges."""
+    rng = np.random.default_rng(nh * 100 + hs)
+    edges = [T for T in range(1, 1100) if _one_kernel(nh, nkv, hs, T, kv_f16) != _one_kernel(nh, nkv, hs, T + 1, kv_f16)]
+    assert len(edges) == (1 if hs % 16 == 0 else 0)
+    for T in edges or [256]:
+        for n in (T, T + 1):
+            got, ref = _attn_case(ctx, nh, nkv, hs, n, n - 1, kv_f16, rng)
+            assert np.abs(got - ref).max() <= 1e-5, f"{n} positions"
+
+
+@pytest.mark.timeout(300)
+@pytest.mark.parametrize("use_graph", [True, False])
+@pytest.mark.parametrize("p0,n,host_end", [(100, 3, 256), (1270, 20, 1536), (1526, 20, 1792)])
+def test_decode_past_the_host_bound(ctx, oracle_lib, use_graph, p0, n, host_end):
+    """Steps whose attention takes the one-kernel form (64 dims, up to 256
+    positions) and the split one (across the edges of two buckets), each step
+    against the oracle over the same planted rows; then the device position
+    moved past the host's bound, where the kernels discard the rows they
+    loaded before they knew it: one position past, and thousands."""
+    import inferi_amd as I
+
+    cfg = I.Llama2Config(n_layers=2, hidden=256, ffn=512, n_heads=4, n_kv_heads=1, vocab=1000, max_pos=8000,
+                         rope_theta=10000.0, rms_eps=1e-5, kv_dtype=I.F16)
+    w = I.Llama2Weights.synthetic(ctx, cfg, seed=93, std=0.05)
+    s = I.Llama2State(ctx, cfg)
+    try:
+        m = oracle_model(cfg, w)
+        rng = np.random.default_rng(p0)
+        for layer in range(cfg.n_layers):
+            for name, which in (("key_cache", "k"), ("value_cache", "v")):
+                rows = O.encode_f16(rng.standard_normal((cfg.max_pos, cfg.kv_dim), np.float32))
+                m.set_kv_rows(layer, which, rows)
+                ptr, _ = s.buffer(name, layer)
+                ctx._check(I.lib().ifr_upload(ctx.h, ptr, rows.ctypes.data, rows.nbytes))
+        toks = rng.integers(0, cfg.vocab, cfg.max_pos - 1).astype(np.uint32)
+        s.reset(toks, p0)
+        for pos in range(p0, p0 + n):
+            I.Llama2.generate(ctx, s, w, 1, use_graph=use_graph)
+            assert_close(s.read("logits"), m.forward(int(toks[pos]), pos), what=f"pos {pos}")
+        for far in (host_end, 5000):  # position host_end is row host_end + 1: one past the bucket's rows
+            s.reset(toks, p0 + n)
+            ptr, _ = s.buffer("pos")
+            jump = np.array([far], np.uint32)
+            ctx._check(I.lib().ifr_upload(ctx.h, ptr, jump.ctypes.data, 4))
+            I.Llama2.generate(ctx, s, w, 1, use_graph=use_graph)
+            assert_close(s.read("logits"), m.forward(int(toks[far]), far), what=f"pos {far}")
+    finally:
+        s.close()
+        w.close()
