@@ -178,10 +178,10 @@ struct ifr_ctx {
         auto it = fns.find(name);
         if (it != fns.end()) return it->second;
         hipFunction_t f = nullptr;
-        if (hipModuleGetFunction(&f, module, name.c_str()) != hipSuccess) {
-            f = nullptr;
-            hipGetLastError(); // a form that a type does not have: not left for the program's next HIP call
-        }
+        // asked only for kernels that the code object has: a failed look-up
+        // would set the thread's last HIP error, and clearing that one would
+        // take away an error that the program itself left there
+        if (hipModuleGetFunction(&f, module, name.c_str()) != hipSuccess) f = nullptr;
         fns[name] = f;
         return f;
     }
@@ -230,12 +230,14 @@ struct ifr_ctx {
 // ------------------------------------------------------------------ GEMV --
 
 struct GemvPlan {
+    int32_t dtype;
     const char *fmt;
     uint32_t nb, row_bytes;
     uint32_t bpi; // blocks per integer-path step (int_blocks_per_step)
 };
 
 static ifr_status check_gemv(ifr_ctx *c, int32_t dtype, uint32_t cols, const void *w, GemvPlan &p) {
+    p.dtype = dtype;
     p.fmt = gemv_fmt_name(dtype);
     if (!p.fmt) return c->fail(IFR_EUNSUPPORTED, "matmul_quant: dtype %d has no GEMV kernel", dtype);
     const int qk = gemv_qk(dtype);
@@ -309,10 +311,10 @@ static ifr_status launch_gemv(ifr_ctx *c, const GemvPlan &p, const char *mode, G
     // workgroup launched at once
     const bool one_mode = !strcmp(mode, "plain") || !strcmp(mode, "qkv");
     if (one_mode && a.nb <= p.bpi && !c->gemv_waves && !c->gemv_max_grid && a.total_rows) {
-        // four rows per wave where the code object has that form (bit 8;
-        // slower for the QKV launch's 6144 rows, whose 384 workgroups of
-        // four-row waves do not fill the chip)
-        const bool four = (c->gemv_grp & 256) && c->fn(name + "_one4");
+        // four rows per wave (bit 8; Q4_K's form; slower for the QKV launch's
+        // 6144 rows, whose 384 workgroups of four-row waves do not fill the
+        // chip)
+        const bool four = (c->gemv_grp & 256) && p.dtype == IFR_Q4_K;
         const uint32_t rows_per = GEMV_ONE_WAVES * (four ? 4 : 2), g = (a.total_rows + rows_per - 1) / rows_per;
         a.ks = 1;
         a.nwaves = GEMV_ONE_WAVES;
@@ -320,19 +322,17 @@ static ifr_status launch_gemv(ifr_ctx *c, const GemvPlan &p, const char *mode, G
         return c->launch(name + (four ? "_one4" : "_one"), dim3(g), dim3(GEMV_ONE_WAVES * 64),
                          (uint32_t)xq_bytes(a.cols), a);
     }
-    // resid and gateup: one output group per workgroup, one item per wave,
-    // where the code object has the form for this format and K
+    // resid and gateup: one output group per workgroup, one item per wave
+    // (Q4_K's forms)
     const bool resid = !strcmp(mode, "resid"), gateup = !strcmp(mode, "gateup");
-    if ((resid || gateup) && !c->gemv_waves && !c->gemv_max_grid && a.total_rows) {
+    if ((resid || gateup) && p.dtype == IFR_Q4_K && !c->gemv_waves && !c->gemv_max_grid && a.total_rows) {
         const uint32_t steps = (a.nb + p.bpi - 1) / p.bpi;
-        char kn[96] = {0};
+        const char *kn = nullptr;
         const bool alt = c->gemv_grp & 8;
-        if (resid && steps == 1 && (c->gemv_grp & 1)) snprintf(kn, sizeof kn, "gemv_%s_resid_r2w8k1", p.fmt);
-        else if (resid && steps > 1 && steps <= 4 && (c->gemv_grp & 2)) snprintf(kn, sizeof kn, "gemv_%s_resid_r4w4k4", p.fmt);
-        else if (gateup && steps == 1 && (c->gemv_grp & 4))
-            snprintf(kn, sizeof kn, alt ? "gemv_%s_gateup_r2w16k1" : "gemv_%s_gateup_r4w8k1", p.fmt);
-        hipFunction_t f = kn[0] ? c->fn(kn) : nullptr;
-        if (f) {
+        if (resid && steps == 1 && (c->gemv_grp & 1)) kn = "gemv_q4_k_resid_r2w8k1";
+        else if (resid && steps > 1 && steps <= 4 && (c->gemv_grp & 2)) kn = "gemv_q4_k_resid_r4w4k4";
+        else if (gateup && steps == 1 && (c->gemv_grp & 4)) kn = alt ? "gemv_q4_k_gateup_r2w16k1" : "gemv_q4_k_gateup_r4w8k1";
+        if (kn) {
             const uint32_t gr = gateup ? 32 : 16, g = (a.total_rows + gr - 1) / gr;
             const uint32_t waves = resid && steps == 1 ? 8 : resid ? 16 : alt ? 16 : 8;
             a.ks = steps;
@@ -345,10 +345,10 @@ static ifr_status launch_gemv(ifr_ctx *c, const GemvPlan &p, const char *mode, G
     a.ks = g.ks;
     a.nwaves = g.waves;
     if (grid_out) *grid_out = g.grid;
-    // the head's form with up to 256 VGPRs, where the code object has it:
-    // two workgroups per CU, each looping over its share of the row groups
-    // (measured fastest: 3 or 4 per CU and the 128-VGPR form are slower)
-    if (!strcmp(mode, "head") && (c->gemv_grp & 64) && g.waves <= 4 && !c->gemv_max_grid && c->fn(name + "_w2")) {
+    // the head's form with up to 256 VGPRs (Q6_K's): two workgroups per CU,
+    // each looping over its share of the row groups (measured fastest: 3 or 4
+    // per CU and the 128-VGPR form are slower)
+    if (!strcmp(mode, "head") && p.dtype == IFR_Q6_K && (c->gemv_grp & 64) && g.waves <= 4 && !c->gemv_max_grid) {
         const uint32_t gg = std::min(g.grid, (uint32_t)c->n_cu * 2);
         if (grid_out) *grid_out = gg;
         return c->launch(name + "_w2", dim3(gg), dim3(g.waves * 64), (uint32_t)xq_bytes(a.cols), a);
@@ -941,7 +941,7 @@ static ifr_status enqueue_head(ifr_ctx *c, ifr_llama2_state *s, const ifr_llama2
         // one item per wave and a key per workgroup when the state holds them
         const uint32_t one_grid = (cfg.vocab + GEMV_ONE_WAVES * 2 - 1) / (GEMV_ONE_WAVES * 2);
         const std::string one = std::string("gemv_") + p.fmt + "_head_one";
-        if ((c->gemv_grp & 16) && !c->gemv_exact && p.nb <= p.bpi && one_grid <= s->part_keys_cap && c->fn(one)) {
+        if ((c->gemv_grp & 16) && !c->gemv_exact && p.nb <= p.bpi && one_grid <= s->part_keys_cap) {
             a.ks = 1;
             a.nwaves = GEMV_ONE_WAVES;
             if ((st = c->launch(one, dim3(one_grid), dim3(GEMV_ONE_WAVES * 64), (uint32_t)xq_bytes(a.cols), a))) return st;

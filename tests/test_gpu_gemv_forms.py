@@ -126,3 +126,43 @@ def test_ffn_f32_hidden_every_type(ctx, gate, down, hidden, ffn):
         w.close()
     err = np.abs(logits[True] - logits[False]).max() / np.abs(logits[False]).max()
     assert err <= 1e-4, f"{err:.2e}"
+
+
+@pytest.mark.parametrize("planted", [False, True])
+def test_choosing_a_form_leaves_hip_errors_alone(planted):
+    """Forms that a type does not have (the grouped and four-row ones but for
+    Q4_K, the head's 256-VGPR one but for Q6_K) are not asked of the HIP
+    runtime: neither an error of a failed look-up is left to the program's
+    next HIP check, nor one taken away that the program itself left (a
+    device that does not exist)."""
+    import ctypes
+
+    import inferi_amd as I
+
+    ctx = I.LlmContext(0)  # its own: a context looks a kernel up once
+    path = next(ln.split()[-1] for ln in open("/proc/self/maps") if "libamdhip64.so" in ln)
+    hip = ctypes.CDLL(path)
+    cfg = I.Llama2Config(n_layers=1, hidden=256, ffn=512, n_heads=4, n_kv_heads=2, vocab=64, max_pos=8,
+                         rope_theta=10000.0, rms_eps=1e-5, kv_dtype=I.F16)
+    w = I.Llama2Weights.synthetic(ctx, cfg, seed=1, mat_dtype=I.Q8_0, head_dtype=I.Q8_0, embd_dtype=I.Q8_0)
+    s = I.Llama2State(ctx, cfg)
+    x, xq, y = ctx.zeros(1024), ctx.alloc(ctx.activation_bytes(256)), ctx.alloc(4096)
+    try:
+        hip.hipGetLastError()
+        if planted:
+            assert hip.hipSetDevice(-1) != 0
+        ctx.quantize_activation(xq, x, 256)  # what an ordinary call leaves of it
+        before = hip.hipPeekAtLastError()
+        for grp in (511, 225):
+            ctx.set_option("gemv_grp", grp)
+            s.reset([1, 2], 0)
+            I.Llama2.launch(ctx, s, w)
+            ctx.matmul_quant_xq(y, x, I.F32, 1, 256, xq)
+            assert hip.hipPeekAtLastError() == before
+    finally:
+        hip.hipGetLastError()
+        s.close()
+        w.close()
+        for b in (x, xq, y):
+            b.free()
+        ctx.close()
