@@ -63,9 +63,10 @@ def test_gemv_forms_same_results(ctx, grp):
 
 @pytest.mark.parametrize("dtype_name,rows,cols", [("Q4_K", 4096, 4096), ("Q4_K", 300, 1024), ("Q6_K", 512, 2048)])
 def test_matmul_quant_four_row_form(ctx, dtype_name, rows, cols):
-    """ifr_matmul_quant with gemv_grp bit 8 (the four-rows-per-wave one-item
-    kernel where the format has one) against the default form, bit for bit,
-    and against the oracle's f64 GEMV at 1e-3."""
+    """gemv_grp bit 8: ifr_matmul_quant_xq takes the four-rows-per-wave one-item
+    kernel where the format has one, ifr_matmul_quant (which quantizes its
+    input in the kernel) its usual one; both against the default form, bit
+    for bit, and against the oracle's f64 GEMV at 1e-3."""
     import inferi_amd as I
     import oracle as O
 
@@ -73,21 +74,24 @@ def test_matmul_quant_four_row_form(ctx, dtype_name, rows, cols):
     rng = np.random.default_rng(rows + cols)
     w = O.quantize(dtype, (rng.standard_normal(rows * cols) * 0.02).astype(np.float32))
     x = rng.standard_normal(cols).astype(np.float32)
-    dw, dx, y = ctx.upload(w), ctx.upload(x), ctx.alloc(rows * 4)
+    dw, dx, y, xq = ctx.upload(w), ctx.upload(x), ctx.alloc(rows * 4), ctx.alloc(ctx.activation_bytes(cols))
     try:
-        ctx.matmul_quant_assign(y, dw, dtype, rows, cols, dx)
-        ref = y.download(np.float32, rows)
-        ctx.set_option("gemv_grp", 225 | 256)
-        try:
-            ctx.matmul_quant_assign(y, dw, dtype, rows, cols, dx)
-        finally:
-            ctx.set_option("gemv_grp", 225)
-        got = y.download(np.float32, rows)
-        assert_same(got, ref, f"{dtype_name} {rows}x{cols}")
+        ctx.quantize_activation(xq, dx, cols)
         e = O.gemv_quant(dtype, w, rows, cols, x)
-        assert np.all(np.abs(got - e) <= 1e-3 * np.maximum(np.abs(e), 1.0))
+        for call, arg in ((ctx.matmul_quant_assign, dx), (ctx.matmul_quant_xq, xq)):
+            call(y, dw, dtype, rows, cols, arg)
+            ref = y.download(np.float32, rows)
+            y.upload(np.full(rows, np.nan, np.float32))
+            ctx.set_option("gemv_grp", 225 | 256)
+            try:
+                call(y, dw, dtype, rows, cols, arg)
+            finally:
+                ctx.set_option("gemv_grp", 225)
+            got = y.download(np.float32, rows)
+            assert_same(got, ref, f"{dtype_name} {rows}x{cols}")
+            assert np.all(np.abs(got - e) <= 1e-3 * np.maximum(np.abs(e), 1.0))
     finally:
-        for b in (dw, dx, y):
+        for b in (dw, dx, y, xq):
             b.free()
 
 
