@@ -257,15 +257,43 @@ def test_set_sampler_rejects(ctx):
         w.close()
 
 
-@pytest.mark.parametrize("c", [1, 2, 8191, 8192, 8193])
-def test_sample_topp_group_sizes(ctx, oracle_lib, c):
-    """A crossing group of c distinct probabilities, on both sides of the
-    8192 keys that stay in LDS from the truncation's search to the choice's,
-    between groups of a few higher and many lower ones."""
+def _group_case(c, n=40000):
+    """Logits whose probabilities hold one level-0 bucket (bits 30..20) of
+    exactly c values between fewer higher and many lower ones; returns them
+    shuffled, with the mass above the group and the group's own."""
     rng = np.random.default_rng(c)
-    x = np.full(40000, -9.0, np.float32)
-    x[:c] = (np.arange(c) * (0.05 / c)).astype(np.float32)  # within one bucket or two neighbours
-    x[c : c + 3] = 0.5
-    x = x[rng.permutation(x.size)]
-    for topp in (0.3, 0.9):
+    spread = 0.03 if c > 2 else 0.001
+    g = np.exp(np.arange(c) * (spread / c))
+    p0 = 1.2 * 2.0 ** round(np.log2(0.35 / c / 1.2))  # 1.2 .. 1.2 e^0.03 lie in one bucket, [1.125, 1.25) x 2^k
+    s = 1.0 / p0
+    n_top = 1 if c <= 2 else 3
+    low = (s - 0.4 * s - g.sum()) / (n - c - n_top)
+    x = np.concatenate([np.log(g), np.full(n_top, np.log(0.4 * s / n_top)), np.full(n - c - n_top, np.log(low))])
+    return x[rng.permutation(n)].astype(np.float32), 0.4, float(g.sum() / s)
+
+
+def _bucket(p):
+    return np.asarray(p, np.float32).view(np.uint32) >> 20
+
+
+@pytest.mark.parametrize("c", [1, 2, 100, 8191, 8192, 8193])
+def test_sample_topp_group_sizes(ctx, oracle_lib, c):
+    """A group of c probabilities in one bucket, on both sides of the 8192
+    keys that stay in LDS from the truncation's search to the choice's: the
+    truncation in it and the choice in it or in the group above, and the
+    truncation in the (larger) group below with the choice in any."""
+    x, above, mass = _group_case(c)
+    n = x.size
+    for topp, trunc_in_group in ((above + 0.6 * mass, True), ((above + mass + 1.0) / 2, False)):
         check_case(ctx, x, 1.0, topp, COINS)
+        idx, p = run_sample(ctx, x, 1.0, topp, COINS)
+        cutoff = np.float32(np.float32(1.0) - np.float32(topp)) / np.float32(n - 1)
+        cand = np.sort(p[p >= cutoff])[::-1]
+        crossing = cand[int(np.argmax(np.cumsum(cand.astype(np.float64)) > topp))]
+        in_group = int((_bucket(cand) == _bucket(crossing)).sum())
+        if trunc_in_group:
+            assert in_group == c
+        else:
+            assert in_group == n - c - (1 if c <= 2 else 3)
+        chosen = set(_bucket(p[idx]).tolist())
+        assert len(chosen) >= 2 and (_bucket(crossing) in chosen)
