@@ -178,9 +178,9 @@ def test_c5_prefill_4095_tokens(ctx, oracle_lib):
     against the exact arithmetic within the f16 rounding bound; every layer's
     rows (2e-2 normwise) and the next step's logits (5e-2 scaled: 32 layers of
     f16-operand products) against sequential decode of the same prompt on the
-    device; and passes of 512 tokens (128 x 128 GEMM tiles, where the
-    4095-token pass takes 256 x 256 tiles) give the same rows and logits bit
-    for bit."""
+    device; and passes of 512 tokens (64 to 256 wide GEMM tiles by the
+    product, where the 4095-token pass takes 256 x 256 ones) give the same
+    rows and logits bit for bit."""
     import inferi_amd as I
 
     P = 4096

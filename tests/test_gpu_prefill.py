@@ -1,8 +1,8 @@
 """GPU parity of the prompt (prefill) path.
 
 ifr_gemm_quant multiplies f16 activations by weights of any quantized GGUF
-type dequantized to f16 tiles on the matrix cores, in 256 x 256 or 128 x 128
-tiles (option pf_tile): both forms are checked against an f64 product of the
+type dequantized to f16 tiles on the matrix cores, in 256 x 256 or smaller
+tiles (option pf_tile): the forms are checked against an f64 product of the
 same f16-rounded operands (only the f32 accumulation order may differ) and
 against each other (bit for bit).
 
@@ -35,12 +35,12 @@ def synthetic_q(ctx, rows, cols, seed, dtype):
     return w
 
 
-# (pf_tile, pf_ws): the 128 x 128 form, the 256 x 256 eight-wave form and
-# the 256 x 256 warp-specialized form (Q4_K only; other types ignore pf_ws)
-TILE_FORMS = ((128, 0), (256, 0), (256, 1))
+# (pf_tile, pf_ws): the 128 x 128 form, the 256 x 256 warp-specialized form and
+# the 256 x 256 eight-wave form (Q4_K's; other types ignore pf_ws)
+TILE_FORMS = ((128, 1), (256, 1), (256, 0))
 
 
-def _gemm_case(ctx, dtype, rows, cols, m, w, rng, forms=TILE_FORMS):
+def _gemm_case(ctx, dtype, rows, cols, m, w, rng):
     """y = x . deq(W)^T in each tile form against the f64 product of the same
     f16-rounded operands (bound 2e-5 * sum |x w|), then the accumulating form;
     the tile forms agree bit for bit."""
@@ -48,7 +48,7 @@ def _gemm_case(ctx, dtype, rows, cols, m, w, rng, forms=TILE_FORMS):
 
     outs = []
     ws0 = ctx.get_option("pf_ws")
-    for tile, ws in forms:
+    for tile, ws in TILE_FORMS if dtype == I.Q4_K else TILE_FORMS[:2]:
         ctx.set_option("pf_tile", tile)
         ctx.set_option("pf_ws", ws)
         try:
@@ -104,7 +104,7 @@ FMTS = ["Q4_0", "Q4_1", "Q5_0", "Q5_1", "Q8_0", "Q4_K", "Q5_K", "Q6_K", "Q8_K", 
 @pytest.mark.parametrize("fmt", FMTS)
 @pytest.mark.parametrize("rows,cols,m", [(300, 512, 70), (130, 2048, 129), (300, 512, 300), (130, 2048, 260)])
 def test_gemm_quant_every_format(ctx, oracle_lib, fmt, rows, cols, m):
-    """Each GGUF type's tile loader in both tile forms: quantized synthetic
+    """Each GGUF type's tile loader in its tile forms: quantized synthetic
     weights and raw random blocks with a quarter of the scales subnormal (the
     reference's GEMV test generator, gemv_quant.rs:354-430)."""
     import inferi_amd as I
@@ -473,3 +473,35 @@ def test_prefill_short_prompt_forms(ctx, mat, kv, bias, n):
         w.close()
     for key in ((0, 0), (256, 0)):
         _same(out[0, 1], out[key], f"tile {key[0]}, fuse {key[1]}")
+
+
+@pytest.mark.timeout(300)
+def test_gemm_quant_rows_past_32_bit_offsets(ctx):
+    """Rows of 2^24 halves: the 128 x 128 form's offsets within a tile do not
+    fit 32 bits and its launch is split by rows (127 and 3 here), where a 32 x
+    32 tile's still fit.  Stored and accumulated, the same bits."""
+    import inferi_amd as I
+
+    rows, cols, m = 16, 1 << 24, 130
+    w = synthetic_q(ctx, rows, cols, 1, I.Q4_0)
+    base = np.random.default_rng(2).standard_normal(cols + m, np.float32).astype(np.float16)
+    dx = ctx.alloc(m * cols * 2)
+    for r in range(m):
+        dx.upload(base[r : r + cols], r * cols * 2)
+    y = ctx.alloc(m * rows * 4)
+    out = []
+    try:
+        for tile in (0, 128):
+            ctx.set_option("pf_tile", tile)
+            y.upload(np.full(m * rows, np.nan, np.float32))
+            ctx.gemm_quant(y, w, I.Q4_0, rows, cols, dx, m)
+            a = y.download(np.uint32, m * rows)
+            ctx.gemm_quant(y, w, I.Q4_0, rows, cols, dx, m, accumulate=True)
+            out.append((a, y.download(np.uint32, m * rows)))
+    finally:
+        ctx.set_option("pf_tile", 0)
+        for b in (w, dx, y):
+            b.free()
+    assert np.isfinite(out[0][0].view(np.float32)).all()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)

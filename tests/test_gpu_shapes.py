@@ -196,9 +196,10 @@ def test_decode_model_shapes(ctx, oracle_lib, name, mode):
 def test_prefill_model_shapes(ctx, oracle_lib, name, tile):
     """A 150-token prompt: 149 tokens through ifr_llama2_prefill, then 12
     decode steps, every step's logits and every layer's KV rows against the
-    oracle over the same sequence; with the GEMM tiles chosen by shape (128 x
-    128 here) and forced to 256 x 256 (stacked QKV products with biases and
-    NeoX pairs, odd query groups, rows and tokens past the matrix edges)."""
+    oracle over the same sequence; with the GEMM tiles chosen by shape (32 to
+    256 wide here, by the product) and forced to 256 x 256 (stacked QKV
+    products with biases and NeoX pairs, odd query groups, rows and tokens past
+    the matrix edges)."""
     import inferi_amd as I
 
     P, N = 150, 12
