@@ -106,9 +106,9 @@ IFR_DEV void q4k_store_part(const u32x4_a16 &qv, const Q4kAffine &f, uint32_t p,
 // rounding, with the code's conversion folded into the mixed-precision FMA
 // (v_fma_mix_f32 reads the half in place).  Masks take two codes per
 // instruction, one in each half; f16 subnormal inputs are kept (the default
-// f16 denormal mode).  x exchanges chunks (device/pf_small.h).
-IFR_DEV void q4k_store_part_mix(const u32x4_a16 &qv, const Q4kAffine &f, uint32_t p, _Float16 *tile, uint32_t r,
-                                uint32_t x = 0) {
+// f16 denormal mode).  The whole tile's rows, one thread each, and the half
+// tile's take it; the other forms run the same arithmetic as PgRun<Q4_K>.
+IFR_DEV void q4k_store_part_mix(const u32x4_a16 &qv, const Q4kAffine &f, uint32_t p, _Float16 *tile, uint32_t r) {
     const float dl = f.d1 * 0x1p24f, dh = f.d2 * 0x1p20f; // exact: powers of two
     const uint32_t q[4] = {qv.x, qv.y, qv.z, qv.w};
     uint32_t lo[8], hi[8];
@@ -125,8 +125,8 @@ IFR_DEV void q4k_store_part_mix(const u32x4_a16 &qv, const Q4kAffine &f, uint32_
     }
 #pragma unroll
     for (int c = 0; c < 2; c++) {
-        *(uint4 *)(tile + pg_swz(r, (2 * p + (uint32_t)c) ^ x)) = make_uint4(lo[4 * c], lo[4 * c + 1], lo[4 * c + 2], lo[4 * c + 3]);
-        *(uint4 *)(tile + pg_swz(r, (4 + 2 * p + (uint32_t)c) ^ x)) = make_uint4(hi[4 * c], hi[4 * c + 1], hi[4 * c + 2], hi[4 * c + 3]);
+        *(uint4 *)(tile + pg_swz(r, 2 * p + (uint32_t)c)) = make_uint4(lo[4 * c], lo[4 * c + 1], lo[4 * c + 2], lo[4 * c + 3]);
+        *(uint4 *)(tile + pg_swz(r, 4 + 2 * p + (uint32_t)c)) = make_uint4(hi[4 * c], hi[4 * c + 1], hi[4 * c + 2], hi[4 * c + 3]);
     }
 }
 struct PgHalfQ4K {
@@ -369,14 +369,14 @@ __device__ __attribute__((always_inline)) void pf_gemm_body(const PfGemmArgs &a)
 }
 
 // The store epilogue of the stacked Q | K | V product with the RoPE and
-// KV-cache store fused (a.rope, warp-specialized form, pairs (2i, 2i + 1)):
-// what the store epilogue and pf_rope_kv_k together do, bit for bit.  Column
+// KV-cache store fused (a.rope, pairs (2i, 2i + 1), every form but the
+// eight-wave one): what the store epilogue and pf_rope_kv_k together do, bit for bit.  Column
 // n is element e of q (n < n1), k (n < n2) or v; its bias is added, then q
 // and k rotate with the pair partner, column n ^ 1, held by lane ^ 1 (the
 // accumulator's columns are the lanes, and q, k and v start at even
 // columns), with the (cos, sin) of the row's position and theta_(e mod hs)/2
 // from the pass's table; q goes to Y, k and v to the cache rows of positions
-// p0 + m.  Eight rows at a time: their table loads go out together from
+// p0 + m.  Four rows at a time: their table loads go out together from
 // rows clamped below M.
 template <int MI, int NJ = 2>
 IFR_DEV void pg_epilogue_rope(const PfGemmArgs &a, const float16v (&acc)[MI][NJ], uint32_t lane, uint32_t wm,

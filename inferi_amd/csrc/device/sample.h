@@ -413,7 +413,9 @@ struct SmpCtx {
 // the passes over a group between them: at 128256 elements 19.8 us with
 // ds_bpermute scans, a third barrier, a search of its own for a group's start
 // and the group read twice, 16.5 us as it stands.  One loop over the levels
-// in place of a pass written out for each was smaller and took 21.9 us.
+// in place of a pass written out for each was smaller and took 21.9 us.  The
+// sixteen totals and counts that every thread reads here, unrolled, take the
+// kernel to 128 VGPRs with 2 of them spilled (12 bytes of scratch).
 IFR_DEV int32_t block_first_exceeding(SmpCtx &X, uint64_t v0, uint64_t v1, uint64_t t, uint64_t &excl, uint64_t &total,
                                       uint32_t c0, uint32_t c1, uint32_t &cnt) {
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;

@@ -50,7 +50,10 @@ using namespace ifr;
 // instruction caches (64 KB per two CUs) hold from one step to the next if
 // they do not fall on the same sets.  Wherever the rest of the code object
 // had put them before, the same step took 493.5 to 499.5 us on the 8B widths
-// with eight layers (as other kernels were added), here 493.
+// with eight layers (as other kernels were added), here 493.  It is that step's
+// order only (128-dim heads in groups of four past the one-kernel attention's
+// contexts): the kernels of other types, head sizes and short contexts lie where
+// the rest of the file puts them; what that costs their steps was not measured.
 extern "C" __global__ void __launch_bounds__(256) embed_k(EmbedArgs a) { embed_body(a); }
 GEMV_ONE_KERNEL(gemv_q4_k_qkv, Q4_K, GEMV_QKV)
 extern "C" __global__ void __launch_bounds__(256) attn_f16_h128_g4(AttnArgs a) { attn_split_body<128, 4, true>(a); }
